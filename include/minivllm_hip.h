@@ -113,15 +113,17 @@ int mgi_kv_append(void* k_pool, void* v_pool,
  * online_v1 result for a row with no active block).
  * q, out and the pool share one dtype; arithmetic is fp32.
  *
- * split_tokens: 0 lets the library split the work. When a table is wider
- * than one partition and B <= 4096 it splits evenly: the blocks of all
+ * split_tokens: 0 lets the library split the work. Small calls give each
+ * (sequence, head) to one workgroup, in one launch and without using the
+ * workspace. Otherwise, when a table is wider
+ * than one partition and B <= 4096, it splits evenly: the blocks of all
  * sequences, in sequence order, are cut into equal segments, one per
  * wavefront of a fixed count (mgi_paged_decode_balanced_waves), whatever the
  * spread of context lengths; each wavefront streams most of its segment and
  * the rest of every segment goes, in small runs, to whichever wavefronts
  * finish first. Otherwise, and for split_tokens > 0 (rounded to a multiple
- * of S), each context is cut into partitions of split_tokens tokens. Either
- * way, a sequence whose work is split writes (max, sum, unnormalised output)
+ * of S), each context is cut into partitions of split_tokens tokens. In both
+ * splits, a sequence whose work is split writes (max, sum, unnormalised output)
  * partials that a second pass merges. The output does not depend on which
  * wavefront streams which run: calls with the same inputs give the same
  * bits.
@@ -228,9 +230,10 @@ int64_t mgi_paged_decode_split_tokens(int64_t B, int64_t H, int64_t D,
                                       int64_t S, int64_t M,
                                       int64_t split_tokens);
 
-/* Wavefronts per group of heads of the even split mgi_paged_decode uses for
- * these sizes on the current device, or 0 when it splits into partitions
- * (or does not split). No counterpart in the reference: it reports the
+/* Wavefronts per group of heads of the even split for these sizes on the
+ * current device (what mgi_paged_decode uses unless the call is small enough
+ * for one workgroup per (sequence, head)), or 0 when it splits into
+ * partitions (or does not split). No counterpart in the reference: it reports the
  * split, as mgi_paged_decode_split_tokens does. */
 int64_t mgi_paged_decode_balanced_waves(int64_t B, int64_t H, int64_t D,
                                         int64_t S, int64_t M,

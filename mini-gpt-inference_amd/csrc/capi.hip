@@ -149,6 +149,46 @@ SplitPlan split_plan(int64_t B, int64_t H, int64_t D, int64_t S, int64_t M, int6
   return sp;
 }
 
+// Wavefronts per workgroup of the workgroup kernel (paged_decode_wg: one
+// workgroup per (sequence, head), one launch), or 0 to use the split chosen
+// above. It saves the context scan, the partials and the merge launch,
+// about 8 us; it loses where one workgroup's context is long (a CU alone
+// streams about 46 KB/us, and the longest context ends the call), on large
+// calls (its one-head pieces stream at 6.2 TB/s against 6.7, 64-byte ones
+// at 3.5) and where launching many short workgroups costs more than their
+// work (about 1.2 ns per wavefront). Balanced groups of 64 / LPH heads that
+// H does not fill stream at 1.25 times the filled share, at most all, of
+// their rate. Calls whose table fits one partition had one wavefront walk
+// each context alone, 0.14 us per token (0.18 in f32). The terms below are
+// those costs in us, for contexts that fill the table. Measured on MI355X
+// (us, without / with; bf16, D = 128 unless noted): 4 sequences x 8 heads,
+// D = 32, contexts 200-256, f32: 48 / 6.4; 13 x 16, 100-1000: 25.2 / 18.9;
+// 16 x 16, 256-768: 26.2 / 17.1; 32 x 8, 128-1024: 27.6 / 19.7; 128 x 16, D
+// = 64, 64-512: 37.0 / 34.3; 20 x 16, D = 96, 200-250: 42.8 / 11.7; 190 x
+// 4, D = 64, 4861-9723: 345 / 259; 139 x 2, 5262: 190 / 166. Kept on the
+// splits: 1 x 32 at 2000: 20.4 / 26.8; 4 x 32 at 4000: 52.7 / 56.1; 64 x 4,
+// 512-4096: 58.0 / 62.0; 256 x 32, 128-2048: 730 / 765; 256 x 16, D = 64,
+// 10-100: 14.7 / 21.6; 49 x 30, D = 32, 4642: 147 / 254; 53 x 2, D = 96,
+// 8085, f32: 175 / 199. Eight wavefronts, except four where a context is at
+// most half a step of the eight, or two steps on a large grid (22 x 22,
+// 29-59: 6.7 against 7.7; 200 x 8, D = 64, 16-512: 27.2 against 29.8).
+// MINIVLLM_HIP_DECODE_WG = 0 turns the kernel off, 4 or 8 forces it (tuning
+// and tests; read on every call).
+int wg_waves_for(int64_t B, int64_t H, int64_t D, int64_t S, int64_t M, int64_t eb, bool split) {
+  const int forced = env_int("MINIVLLM_HIP_DECODE_WG", -1);
+  if (forced >= 0) return forced == 0 ? 0 : forced == 4 ? 4 : 8;
+  const int64_t lph = D <= 32 ? 4 : D <= 64 ? 8 : D <= 128 ? 16 : 32, hpw = 64 / lph;
+  const int64_t step_tokens = 8 * hpw * (mgi::kGranuleLoads * 2 / eb);  // one step of eight wavefronts
+  const bool large_grid = B * H >= 4 * (int64_t)device_cus();
+  const int waves = M * S <= (large_grid ? 2 * step_tokens : step_tokens / 2) ? 4 : 8;
+  const double wg_mb = 2e-6 * (double)(M * S) * (double)(D * eb), all_mb = wg_mb * (double)(B * H);
+  const double filled = (double)H / (double)((H + hpw - 1) / hpw * hpw);  // of the balanced split's lanes
+  const double wg_us = std::max(all_mb / (D <= 32 ? 3.5 : 6.2), 1.2e-3 * (double)(B * H * waves)) + wg_mb * 10.9;
+  const double other_us = split ? 8.0 + all_mb / (6.7 * std::min(1.0, 1.25 * filled))
+                                : std::max(all_mb / 6.7, (eb == 4 ? 0.18 : 0.14) * (double)(M * S));
+  return wg_us < other_us ? waves : 0;
+}
+
 struct WorkspaceLayout {
   size_t acc_bytes, ml_offset, cinc_offset, ticket_offset, total;
 };
@@ -581,6 +621,12 @@ int paged_decode_impl(void* out, const int64_t* out_strides, const void* q,
       a.ws_cinc = reinterpret_cast<int*>(static_cast<char*>(workspace) + ws.cinc_offset);
       a.ws_ticket = reinterpret_cast<int*>(static_cast<char*>(workspace) + ws.ticket_offset);
     }
+  }
+
+  if (plan.path == DecodePath::kFast && split_tokens <= 0) {
+    a.wg_waves = wg_waves_for(B, H, D, S, M, eb, sp.max_parts > 1);
+    const int64_t gpb = S / (kGranuleLoads * 2 / eb);  // granules per block (S is a multiple of the fast step)
+    a.gpb_shift = (gpb & (gpb - 1)) == 0 ? __builtin_ctzll((unsigned long long)gpb) : -1;
   }
 
   if (ap) {

@@ -35,6 +35,8 @@ struct DecodeArgs {
   int bal_tier1_16ths;// balanced mode: share of each segment in its wave's own claim (16ths)
   int bal_tier2;      // balanced mode: ticket claims per segment, at most (0: none)
   int bal_claims;     // balanced mode: bal_waves * (1 + bal_tier2), partial slot pairs per head
+  int wg_waves;       // > 0: one workgroup of this many wavefronts per (sequence, head)
+  int gpb_shift;      // workgroup kernel: log2(granules per block), -1 when not a power of two
   int merge_waves;    // wavefronts per workgroup of paged_decode_merge (1, 2, 4 or 8)
   float* ws_acc;      // [B, H, max_parts, D] unnormalised partial outputs
   float2* ws_ml;      // [B, H, max_parts]    partial (max, sum), log2 domain
@@ -99,6 +101,10 @@ struct PrefillArgs {
   float* ws_acc;      // split keys: [T, H, max_parts, D] unnormalised partial outputs
   float2* ws_ml;      // split keys: [T, H, max_parts] partial (max, sum), log2 domain
 };
+
+// Workgroup decode kernel: 16-byte loads of K (and as many of V) a lane issues
+// per granule of consecutive tokens: 4 tokens of the 2-byte types, 2 of f32.
+constexpr int kGranuleLoads = 4;
 
 // Largest batch of the fast decode kernel's balanced mode (its per-wave
 // prefix sums of blocks per sequence live in LDS).

@@ -19,11 +19,12 @@
 // the log2 domain. Decode attention is HBM-bound (~1 flop/byte), so there is
 // no MFMA and no LDS staging: every lane loads exactly the bytes it consumes.
 //
-// Work split: paged_decode_fast_bal deals the blocks of all sequences out to
+// Work split: paged_decode_wg gives each (sequence, head) to one workgroup
+// (small calls); paged_decode_fast_bal deals the blocks of all sequences out to
 // a fixed number of wavefronts, most of them as each wave's own claim and the
 // rest as small claims that waves draw by ticket once their own is done, so
-// faster XCDs take more (the automatic choice); paged_decode_fast cuts each
-// context into partitions of part_tokens tokens.
+// faster XCDs take more (the automatic choice for large ones);
+// paged_decode_fast cuts each context into partitions of part_tokens tokens.
 // A sequence whose work is split writes (max, sum, unnormalised output)
 // partials that paged_decode_merge combines:
 //   M = max_p m_p,  L = sum_p l_p 2^(m_p - M),  O = sum_p O_p 2^(m_p - M) / L.
@@ -683,6 +684,214 @@ paged_decode_fast_bal(const DecodeArgs a) {
   }
 }
 
+// ------------------------------------------------------- workgroup kernel
+// One workgroup of NW wavefronts per (head, sequence): the whole context in
+// one launch, with no context scan, no partials in memory and no merge launch.
+//
+// The LPH lanes of a row cover one head row as in the fast kernel, but the
+// wavefront's TS = 64 / LPH rows take different tokens of the same head: the
+// context is cut into granules of GT consecutive tokens (S is a multiple of
+// GT, so a granule lies in one block), and row r of the workgroup's NW * TS
+// takes granules r, r + NW * TS, ... Each row keeps its own online softmax
+// state; the rows of a wavefront combine by lane exchange and the wavefronts
+// through LDS. A row's table entry is loaded two steps before its K/V, which
+// are loaded one step before they are folded.
+//
+// Tokens past the context, of masked blocks or of rows with nothing left are
+// read from kDecodeZeroRow and masked, so no slot outside the context is read
+// and its contents cannot reach the sums.
+//
+// Fused append: the row that takes the granule of the sequence's last token
+// writes the new K/V before its first loads; the lanes that load those 16
+// bytes back are the lanes that stored them.
+//
+// What bounds it: on small calls the chain context length -> table entry ->
+// K/V -> merge, about 5 us with its launch (4 sequences x 8 heads, D = 32,
+// 256 tokens, f32: 48 us for one wavefront per 16 heads, 6.1 here); past that
+// what one CU streams alone, about 46 KB/us whether 8 or 16 wavefronts and 4
+// or 8 tokens per granule are in flight (8 tokens: 1-5 % slower at 8
+// wavefronts; 16 wavefronts: 1-10 % slower), and HBM (16 x 16 heads, D = 128,
+// bf16, 256-768 tokens: 26.2 us balanced, 17.1 here, 5.5 TB/s past the
+// launch).
+__device__ __align__(16) const unsigned char kDecodeZeroRow[16] = {0};
+
+typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
+typedef const __attribute__((address_space(1))) char* gbytes;
+
+__device__ __forceinline__ uint4 stream_load16(gbytes p) {
+  return __builtin_bit_cast(uint4,
+                            __builtin_nontemporal_load((const __attribute__((address_space(1))) u32x4*)p));
+}
+
+template <typename T, int LPH, int GT, int NW>
+__global__ void __launch_bounds__(64 * NW)
+paged_decode_wg(const DecodeArgs a) {
+  constexpr int TS = 64 / LPH;   // granules a wavefront takes per step
+  constexpr int NR = NW * TS;    // granules the workgroup takes per step
+  constexpr int NL = Layout<T>::kLoads;
+  constexpr int EB = (int)sizeof(T);
+  constexpr int DMAX = 8 * LPH;
+  __shared__ float st_m[NW], st_l[NW];
+  __shared__ __align__(16) float st_o[NW][DMAX];
+  const int lane = (int)threadIdx.x & 63;
+  const int wv = __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6);
+  const int sub = lane % LPH;
+  const int h = (int)blockIdx.x, b = (int)blockIdx.y;
+  const bool sub_ok = sub * 8 < a.D;
+  const int r0 = wv * TS + lane / LPH;  // this row's first granule
+  const int gpb = a.S / GT;             // granules per block
+  auto block_of = [&](int j) { return a.gpb_shift >= 0 ? j >> a.gpb_shift : j / gpb; };
+
+  QFrag<T> q;
+  load_query<T>(a, b, h, sub, sub_ok, q);
+  const int ctx = clamp_ctx<T>(a, b);
+  const int ngran = (ctx + GT - 1) / GT;
+  const int nsteps = (ngran + NR - 1) / NR;
+  // The table entry of granule j: physical block, -1 when invalid or past the context.
+  const int64_t bt_row = (int64_t)b * a.bt_sb;
+  auto entry = [&](int j) -> int {
+    if (j >= ngran) return -1;
+    const int64_t e = load_index(a.bt, a.bt_i64, bt_row + (int64_t)block_of(j) * a.bt_sm);
+    return (e >= 0 && e < a.N) ? (int)e : -1;
+  };
+  int e0 = entry(r0), e1 = entry(r0 + NR);
+
+  if (a.kw != nullptr) {
+    const int jl = ctx > 0 ? (ctx - 1) / GT : 0;  // an empty sequence's row: the first row
+    if (wv == (jl % NR) / TS) {                   // uniform over the wavefront
+      const int64_t slot = load_index(a.slots, a.sl_i64, (int64_t)b * a.sl_s);
+      if (append_slot_ok(a, slot) && sub_ok && r0 == jl % NR) {
+#pragma unroll
+        for (int j = 0; j < NL; ++j) {
+          uint4 kf, vf;
+          append_load<T>(a, b, h, sub, j, kf, vf);
+          append_store<T>(a, slot, h, sub, j, kf, vf);
+        }
+      }
+      append_fence();
+    }
+  }
+
+  const gbytes kg = (gbytes)a.k, vg = (gbytes)a.v, zero = (gbytes)kDecodeZeroRow;
+  const int64_t k_row = a.k_ss * EB, v_row = a.v_ss * EB;
+  uint32_t koff[NL], voff[NL];
+  row_offsets<T>(a, h, sub, true, koff, voff);
+
+  // Issues the loads of this row's granule of step s (table entry phys);
+  // returns its number of tokens to fold (0: none).
+  auto issue = [&](int s, int phys, Step<T, GT>& st) -> int {
+    const int j = s * NR + r0;
+    int nv = min(GT, ctx - j * GT);
+    if (phys < 0) nv = 0;  // masked, or past the context
+    const int off = (j - block_of(j) * gpb) * GT;
+    const int64_t pb = phys >= 0 ? phys : 0;
+    const gbytes kp = kg + (pb * a.k_sn + (int64_t)off * a.k_ss) * EB;
+    const gbytes vp = vg + (pb * a.v_sn + (int64_t)off * a.v_ss) * EB;
+    const int nl = sub_ok ? nv : 0;
+#pragma unroll
+    for (int t = 0; t < GT; ++t)
+#pragma unroll
+      for (int i = 0; i < NL; ++i) st.k[t][i] = stream_load16(t < nl ? kp + (t * k_row + koff[i]) : zero);
+#pragma unroll
+    for (int t = 0; t < GT; ++t)
+#pragma unroll
+      for (int i = 0; i < NL; ++i) st.v[t][i] = stream_load16(t < nl ? vp + (t * v_row + voff[i]) : zero);
+    return nv;
+  };
+
+  float m = -INFINITY, l = 0.f, acc[8];
+#pragma unroll
+  for (int i = 0; i < 8; ++i) acc[i] = 0.f;
+  auto consume = [&](const Step<T, GT>& st, int nv) {
+#pragma clang fp contract(off)  // as fold_chunk: the largest score's weight is exactly 1
+    float s[GT];
+    float mb = -INFINITY;
+#pragma unroll
+    for (int t = 0; t < GT; ++t) {
+      const float d = group_sum<LPH>(q.dot(st.k[t])) * a.scale_log2;
+      s[t] = t < nv ? d : -INFINITY;
+      mb = fmaxf(mb, s[t]);
+    }
+    const float mn = fmaxf(m, mb);
+    const float mr = (nv == 0 && mn == -INFINITY) ? 0.f : mn;  // a row that has folded nothing yet stays empty
+    const float alpha = fast_exp2(m - mr);
+    float psum = 0.f;
+#pragma unroll
+    for (int i = 0; i < 8; ++i) acc[i] *= alpha;
+#pragma unroll
+    for (int t = 0; t < GT; ++t) {
+      const float p = fast_exp2(s[t] - mr);
+      psum += p;
+#pragma unroll
+      for (int i = 0; i < 8; ++i) acc[i] = fmaf(p, frag_elem<T>(st.v[t], i), acc[i]);
+    }
+    l = l * alpha + psum;
+    m = mn;
+  };
+
+  if (nsteps > 0) {
+    Step<T, GT> A, B;
+    int na = issue(0, e0, A);
+    e0 = entry(r0 + 2 * NR);
+    for (int s = 0; s < nsteps; s += 2) {
+      int nb = 0;
+      if (s + 1 < nsteps) {
+        nb = issue(s + 1, e1, B);
+        e1 = entry(r0 + (s + 3) * NR);
+      }
+      __builtin_amdgcn_sched_barrier(0);
+      consume(A, na);
+      if (s + 1 >= nsteps) break;
+      if (s + 2 < nsteps) {
+        na = issue(s + 2, e0, A);
+        e0 = entry(r0 + (s + 4) * NR);
+      }
+      __builtin_amdgcn_sched_barrier(0);
+      consume(B, nb);
+    }
+  }
+
+  // The rows of the wavefront, then the wavefronts.
+#pragma unroll
+  for (int x = LPH; x < 64; x *= 2) {
+    const float mo = __shfl_xor(m, x, 64), lo = __shfl_xor(l, x, 64);
+    const float mn = fmaxf(m, mo);
+    const float fs = m == -INFINITY ? 0.f : fast_exp2(m - mn);
+    const float fo = mo == -INFINITY ? 0.f : fast_exp2(mo - mn);
+    m = mn;
+    l = l * fs + lo * fo;
+#pragma unroll
+    for (int i = 0; i < 8; ++i) acc[i] = acc[i] * fs + __shfl_xor(acc[i], x, 64) * fo;
+  }
+  if (lane < LPH) {
+    if (lane == 0) {
+      st_m[wv] = m;
+      st_l[wv] = l;
+    }
+    if (sub_ok) {
+      *reinterpret_cast<float4*>(&st_o[wv][Layout<T>::elem(sub, a.D, 0)]) = make_float4(acc[0], acc[1], acc[2], acc[3]);
+      *reinterpret_cast<float4*>(&st_o[wv][Layout<T>::elem(sub, a.D, 4)]) = make_float4(acc[4], acc[5], acc[6], acc[7]);
+    }
+  }
+  __syncthreads();
+  float M = -INFINITY, L = 0.f, f[NW];
+#pragma unroll
+  for (int w = 0; w < NW; ++w) M = fmaxf(M, st_m[w]);
+#pragma unroll
+  for (int w = 0; w < NW; ++w) {
+    f[w] = st_m[w] == -INFINITY ? 0.f : fast_exp2(st_m[w] - M);
+    L = fmaf(f[w], st_l[w], L);
+  }
+  const float inv = L > 0.f ? 1.f / L : 0.f;
+  T* orow = reinterpret_cast<T*>(a.out) + (int64_t)b * a.o_sb + (int64_t)h * a.o_sh;
+  for (int d = (int)threadIdx.x; d < a.D; d += 64 * NW) {
+    float o = 0.f;
+#pragma unroll
+    for (int w = 0; w < NW; ++w) o = fmaf(f[w], st_o[w][d], o);
+    Elem<T>::store(orow + (int64_t)d * a.o_sd, o * inv);
+  }
+}
+
 // Combines the partials of every (b, h) whose context spans more than one
 // piece of work (partition mode: ceil(ctx / part_tokens) partitions;
 // balanced mode: the claims its blocks fall in). One wavefront per (sequence,
@@ -890,6 +1099,15 @@ static hipError_t launch_merge(const DecodeArgs& a, hipStream_t stream) {
   }
 }
 
+template <typename T, int LPH>
+static hipError_t launch_wg(const DecodeArgs& a, hipStream_t stream) {
+  constexpr int GT = kGranuleLoads / Layout<T>::kLoads;
+  const dim3 grid((unsigned)a.H, (unsigned)a.B);
+  if (a.wg_waves == 4)
+    return launch(reinterpret_cast<const void*>(&paged_decode_wg<T, LPH, GT, 4>), grid, dim3(256), a, stream);
+  return launch(reinterpret_cast<const void*>(&paged_decode_wg<T, LPH, GT, 8>), grid, dim3(512), a, stream);
+}
+
 template <typename T, int LPH, int TOK>
 static hipError_t launch_fast_lph_tok(const DecodeArgs& a, bool full, hipStream_t stream) {
   constexpr int HPW = 64 / LPH;
@@ -910,6 +1128,7 @@ static hipError_t launch_fast_lph_tok(const DecodeArgs& a, bool full, hipStream_
 
 template <typename T, int LPH>
 static hipError_t launch_fast_lph(const DecodeArgs& a, const DecodePlan& p, hipStream_t stream) {
+  if (a.wg_waves > 0) return launch_wg<T, LPH>(a, stream);
   if constexpr (sizeof(T) == 2) {
     if (p.tokens_per_step == 16) return launch_fast_lph_tok<T, LPH, 16>(a, p.full_lanes, stream);
     if (p.tokens_per_step == 8) return launch_fast_lph_tok<T, LPH, 8>(a, p.full_lanes, stream);

@@ -1,0 +1,95 @@
+"""The one-launch decode kernel (one workgroup per (sequence, head)) on the
+MI355X: against float64 softmax over the gathered tokens, and its fused append against the split kernels,
+at the sizes where its work division can go wrong -- contexts around a granule
+(4 tokens, 2 in f32), around one and two steps of four and of eight
+wavefronts, empty and one-token contexts, head dims below and at every lane
+layout, block sizes that are not a power of two, masked table entries, and
+NaN in every slot outside a context."""
+from __future__ import annotations
+
+import numpy as np
+import pytest
+import torch
+
+import _fixtures as fx
+from minivllm import hip_paged_decode as hpd
+from test_decode_append_gpu import bits, step_case
+from test_paged_decode_gpu import _small_case, hip
+
+pytestmark = pytest.mark.gpu
+DEV = torch.device("cuda:0")
+# The suite's decode tolerances: f32 sums in another order; one rounding of a
+# 2-byte output of magnitude about one (2^-9 and 2^-12) with room for the order.
+TOL = {torch.float32: 1e-5, torch.bfloat16: 2e-2, torch.float16: 2e-3}
+DTYPES = [torch.float32, torch.bfloat16, torch.float16]
+
+
+def edges(D: int, dtype, waves: int, cap: int) -> list[int]:
+    lph = 4 if D <= 32 else 8 if D <= 64 else 16 if D <= 128 else 32
+    gt = 2 if dtype == torch.float32 else 4
+    step = waves * (64 // lph) * gt
+    ctx = {0, 1, gt - 1, gt, gt + 1, step - 1, step, step + 1, 2 * step, 2 * step + gt + 1, 3 * step - 1, cap}
+    return sorted(c for c in ctx if c <= cap)
+
+
+def reference(q, pool, tables, lens, layer) -> np.ndarray:
+    """softmax(q K^T / sqrt(D)) V in float64 over each row's tokens whose table entry is a block."""
+    S, out = pool.block_size, torch.zeros(q.shape, dtype=torch.float64)
+    for b, n in enumerate(lens.tolist()):
+        phys = tables[b].repeat_interleave(S)[:n]
+        keep = (phys >= 0) & (phys < pool.num_blocks)
+        if not keep.any():
+            continue
+        idx, off = phys[keep], (torch.arange(n) % S)[keep]
+        k, v = pool.k[layer, idx, off].double(), pool.v[layer, idx, off].double()
+        p = torch.softmax((k * q[b].double()).sum(-1) / q.shape[-1] ** 0.5, 0)
+        out[b] = (p.unsqueeze(-1) * v).sum(0)
+    return out.numpy()
+
+
+@pytest.mark.parametrize("waves", [4, 8])
+@pytest.mark.parametrize("dtype", DTYPES)
+@pytest.mark.parametrize("D,S,H", [(8, 16, 3), (32, 16, 8), (64, 8, 5), (80, 24, 2), (128, 16, 4), (256, 40, 1)])
+def test_matches_reference_at_step_edges(D, S, H, dtype, waves, monkeypatch):
+    monkeypatch.setenv("MINIVLLM_HIP_DECODE_WG", str(waves))
+    print(f"  D={D} S={S} H={H} {dtype} waves={waves}", flush=True)
+    ctx = edges(D, dtype, waves, 1100)
+    N = sum((c + S - 1) // S for c in ctx) + 4
+    q, pool, tables, lens, layer = _small_case(len(ctx), H, D, S, ctx, dtype, seed=D + waves, N=N)
+    tables[-1, 1] = -1       # a masked block in the longest context
+    tables[-2, 0] = N + 3    # and an entry past the pool
+    got = hip(q, fx.pool_to_device(pool, DEV), tables, lens, layer)
+    want = reference(q, pool, tables, lens, layer)
+    np.testing.assert_allclose(got, want, atol=TOL[dtype], rtol=TOL[dtype])
+    assert (got[np.array(ctx) == 0] == 0).all()
+
+
+@pytest.mark.parametrize("waves", [4, 8])
+@pytest.mark.parametrize("dtype", DTYPES)
+@pytest.mark.parametrize("D", [32, 96, 128])
+def test_fused_append_matches_two_calls(D, dtype, waves, monkeypatch):
+    """Same pools and outputs, bit for bit, as the append kernel followed by
+    the same attention kernel; the split kernels agree within tolerance."""
+    print(f"  append D={D} {dtype} waves={waves}", flush=True)
+    c = step_case(24, 4, D, 16, 1, 700, dtype, seed=D + waves)
+    pools = [fx.pool_to_device(c["pool"], DEV) for _ in range(2)]
+    monkeypatch.setenv("MINIVLLM_HIP_DECODE_WG", str(waves))
+    fused = hpd.paged_attention_batch_append_hip(c["q"], pools[0], c["tables"], c["ctx"], 1, c["k"], c["v"], c["slots"])
+    hpd.kv_append(pools[1], 1, c["k"], c["v"], c["slots"])
+    two = hpd.paged_attention_batch_hip(c["q"], pools[1], c["tables"], c["ctx"], 1)
+    monkeypatch.setenv("MINIVLLM_HIP_DECODE_WG", "0")
+    split = hpd.paged_attention_batch_hip(c["q"], pools[1], c["tables"], c["ctx"], 1)
+    assert torch.equal(bits(pools[0].k), bits(pools[1].k)) and torch.equal(bits(pools[0].v), bits(pools[1].v))
+    assert torch.equal(bits(fused), bits(two))
+    torch.testing.assert_close(fused, split, atol=TOL[dtype], rtol=TOL[dtype])
+
+
+@pytest.mark.parametrize("dtype", DTYPES)
+def test_split_kernels_still_match_where_the_rule_leaves_them(dtype, monkeypatch):
+    """The shapes the one-launch kernel now takes, on the balanced split."""
+    monkeypatch.setenv("MINIVLLM_HIP_DECODE_WG", "0")
+    ctx = [0, 1, 17, 255, 256, 640]
+    q, pool, tables, lens, layer = _small_case(6, 8, 128, 16, ctx, dtype, seed=9, N=90)
+    got = hip(q, fx.pool_to_device(pool, DEV), tables, lens, layer)
+    want = reference(q, pool, tables, lens, layer)
+    np.testing.assert_allclose(got, want, atol=TOL[dtype], rtol=TOL[dtype])
