@@ -61,7 +61,8 @@ const char* mgi_last_error(void);
  * mgi_paged_decode_balanced_waves and the even split of split_tokens = 0;
  * 1.02 the prefill key split (mgi_paged_prefill's workspace arguments and
  * mgi_paged_prefill_workspace_bytes); 1.03 mgi_paged_decode_noalloc; 1.04
- * mgi_paged_decode_append. */
+ * mgi_paged_decode_append. mgi_decode_linear and mgi_decode_linear_norm came
+ * later without a change to the others. */
 int mgi_abi_version(void);
 
 /*
@@ -288,6 +289,35 @@ int mgi_paged_prefill(void* out, const int64_t* out_strides, /* [3] */
  * mgi_paged_decode_workspace_bytes does for decode. */
 size_t mgi_paged_prefill_workspace_bytes(int64_t start_pos, int64_t T,
                                          int64_t H, int64_t D, int dtype);
+
+/*
+ * One linear layer of a decode step with what follows it in a pre-LN block:
+ *   out[b,:] = act(x[b,:] W^T + bias)
+ * x [B, K], weight [N, K], out [B, N], bias [N], contiguous and 16-byte
+ * aligned, all of one 2-byte dtype. bias may be null; gelu != 0 applies the exact (erf) GELU. Arithmetic is fp32 and the result is
+ * rounded once. B <= 64, K a multiple of 64 up to 2560; other sizes return
+ * MGI_EUNSUPPORTED. out must not overlap the inputs.
+ */
+int mgi_decode_linear(void* out, const void* x, const void* weight, const void* bias,
+                      int gelu, int dtype, int64_t B, int64_t N, int64_t K, void* stream);
+
+/*
+ * The projection back to the residual stream and the LayerNorm that follows:
+ *   out[b,:] = x[b,:] W^T + bias + residual[b,:],  norm[b,:] = LN(out[b,:])
+ * Layouts and dtypes as mgi_decode_linear; any K that is a multiple of 64, N a
+ * multiple of 4 up to 4096, B <= 64. bias may be null; norm, ln_weight and
+ * ln_bias may be null together; with x, weight and out null, norm is the
+ * LayerNorm of residual. K is split over workgroups: workspace holds their f32
+ * sums (mgi_decode_linear_norm_workspace_bytes; contents as
+ * mgi_paged_decode's), which a second launch adds up.
+ */
+int mgi_decode_linear_norm(void* out, void* norm, const void* x, const void* weight, const void* bias,
+                           const void* residual, const void* ln_weight, const void* ln_bias,
+                           float ln_eps, int dtype, int64_t B, int64_t N, int64_t K,
+                           void* workspace, size_t workspace_bytes, void* stream);
+
+/* Workspace bytes mgi_decode_linear_norm needs for these sizes. */
+size_t mgi_decode_linear_norm_workspace_bytes(int64_t B, int64_t N, int64_t K);
 
 #ifdef __cplusplus
 }

@@ -7,6 +7,7 @@
 #include <atomic>
 #include <cmath>
 #include <cstdlib>
+#include <initializer_list>
 #include <mutex>
 #include <string>
 
@@ -474,6 +475,29 @@ int launch_append(const AppendSpec& ap, const int64_t* k_pool_strides, const int
   return MGI_OK;
 }
 
+// Checks the two decode-step linear calls share.
+int check_linear(std::initializer_list<const void*> tensors, int dtype, int64_t B, int64_t N, int64_t K) {
+  using namespace mgi;
+  if (B <= 0 || N <= 0 || K <= 0) return fail(MGI_EINVAL, "dimensions must be nonzero");
+  if (dtype != MGI_BF16 && dtype != MGI_F16) return fail(MGI_EUNSUPPORTED, "decode_linear takes bf16 and f16");
+  if (B > kLinearMaxRows) return fail(MGI_EUNSUPPORTED, "more rows than one decode_linear call takes");
+  if (K % 64 != 0) return fail(MGI_EUNSUPPORTED, "K must be a multiple of 64");
+  if (N >= (int64_t(1) << 30) || K >= (int64_t(1) << 30)) return fail(MGI_EUNSUPPORTED, "weight too large");
+  for (const void* p : tensors)
+    if (!aligned16(p)) return fail(MGI_EUNSUPPORTED, "tensors must be 16-byte aligned");
+  return MGI_OK;
+}
+
+// Splits of K of mgi_decode_linear_norm, and the 64-wide units of each: eight
+// splits, or as many as keep a split's rows of x within 128 KiB of LDS (64
+// rows of 16 units).
+int linear_splits(int64_t K, int* units) {
+  const int64_t n = K / 64;
+  const int64_t per = std::min<int64_t>(16, (n + 7) / 8);
+  if (units) *units = (int)per;
+  return (int)((n + per - 1) / per);
+}
+
 // The body of mgi_paged_decode, mgi_paged_decode_noalloc and
 // mgi_paged_decode_append. With `use_scratch` the workspace is the device's
 // allocation-free scratch (resolved here once the call is known to need it,
@@ -743,6 +767,71 @@ int mgi_kv_append(void* k_pool, void* v_pool, const int64_t* k_pool_strides,
   if (rc != MGI_OK) return rc;
   return launch_append(ap, k_pool_strides, v_pool_strides, pool_dtype, T, H, D, S, N, layer_idx,
                        static_cast<hipStream_t>(stream));
+}
+
+int mgi_decode_linear(void* out, const void* x, const void* weight, const void* bias, int gelu, int dtype,
+                      int64_t B, int64_t N, int64_t K, void* stream) {
+  using namespace mgi;
+  g_err.clear();
+  if (!out || !x || !weight) return fail(MGI_EINVAL, "null tensor pointer");
+  const int rc = check_linear({out, x, weight, bias}, dtype, B, N, K);
+  if (rc != MGI_OK) return rc;
+  if (K > kLinearMaxK) return fail(MGI_EUNSUPPORTED, "K larger than one launch takes");
+  LinearArgs a{};
+  a.x = x;
+  a.w = weight;
+  a.bias = bias;
+  a.out = out;
+  a.B = (int)B;
+  a.N = (int)N;
+  a.K = (int)K;
+  a.gelu = gelu;
+  a.cus = device_cus();
+  const hipError_t e = launch_decode_linear(a, dtype, static_cast<hipStream_t>(stream));
+  if (e != hipSuccess) return fail(MGI_ELAUNCH, std::string("launch failed: ") + hipGetErrorString(e));
+  return MGI_OK;
+}
+
+size_t mgi_decode_linear_norm_workspace_bytes(int64_t B, int64_t N, int64_t K) {
+  if (B <= 0 || N <= 0 || K <= 0) return 0;
+  return (size_t)(linear_splits(K, nullptr) * B * N * 4);
+}
+
+int mgi_decode_linear_norm(void* out, void* norm, const void* x, const void* weight, const void* bias,
+                           const void* residual, const void* ln_weight, const void* ln_bias, float ln_eps,
+                           int dtype, int64_t B, int64_t N, int64_t K, void* workspace, size_t workspace_bytes,
+                           void* stream) {
+  using namespace mgi;
+  g_err.clear();
+  if (!residual || !x != !weight || !x != !out || (!out && !norm)) return fail(MGI_EINVAL, "null tensor pointer");
+  if (!norm != !ln_weight) return fail(MGI_EINVAL, "norm needs the LayerNorm weight and bias");
+  if (!ln_weight != !ln_bias) return fail(MGI_EINVAL, "LayerNorm needs weight and bias");
+  const int rc = check_linear({out, norm, x, weight, bias, ln_weight, ln_bias, residual, workspace}, dtype, B, N,
+                              x ? K : 64);
+  if (rc != MGI_OK) return rc;
+  if (N > kReduceMaxN || N % 4 != 0) return fail(MGI_EUNSUPPORTED, "rows must be at most 4096 wide, a multiple of 4");
+  LinearArgs a{};
+  a.x = x;
+  a.w = weight;
+  a.bias = x ? bias : nullptr;
+  a.gamma = ln_weight;
+  a.beta = ln_bias;
+  a.res = residual;
+  a.out = out;
+  a.norm = norm;
+  a.B = (int)B;
+  a.N = (int)N;
+  a.K = (int)K;
+  a.eps = ln_eps;
+  if (x) {
+    a.splits = linear_splits(K, &a.split_units);
+    if (!workspace || workspace_bytes < mgi_decode_linear_norm_workspace_bytes(B, N, K))
+      return fail(MGI_EWORKSPACE, "workspace smaller than mgi_decode_linear_norm_workspace_bytes()");
+    a.part = static_cast<float*>(workspace);
+  }
+  const hipError_t e = launch_decode_linear_split(a, dtype, static_cast<hipStream_t>(stream));
+  if (e != hipSuccess) return fail(MGI_ELAUNCH, std::string("launch failed: ") + hipGetErrorString(e));
+  return MGI_OK;
 }
 
 int mgi_paged_prefill(void* out, const int64_t* out_strides, const void* q,

@@ -106,6 +106,33 @@ struct PrefillArgs {
 // per granule of consecutive tokens: 4 tokens of the 2-byte types, 2 of f32.
 constexpr int kGranuleLoads = 4;
 
+// Linear layer of a decode step (see decode_linear.hip): contiguous rows, 2-byte
+// types, K a multiple of 64, every pointer 16-byte aligned.
+struct LinearArgs {
+  const void* x;      // [B, K]
+  const void* w;      // [N, K]
+  const void* bias;   // [N] or null
+  void* out;          // [B, N]
+  int B, N, K;
+  int gelu;           // one-launch form
+  int cus;            // one-launch form: compute units of the device
+  // Split form:
+  const void* res;    // [B, N] residual
+  const void* gamma;  // LayerNorm weight and bias [N], or both null
+  const void* beta;
+  void* norm;         // [B, N]: LayerNorm of the result
+  float eps;
+  float* part;        // [splits, B, N] f32 sums
+  int splits;         // splits of K (0: norm of the residual alone)
+  int split_units;    // 64-wide units of K per split
+};
+constexpr int kLinearMaxRows = 64;     // rows a call may have
+constexpr int kLinearMaxK = 2560;      // widest K of the one-launch form
+constexpr int kReduceMaxN = 4096;      // widest row of the split form
+
+hipError_t launch_decode_linear(const LinearArgs& a, int dtype, hipStream_t stream);
+hipError_t launch_decode_linear_split(const LinearArgs& a, int dtype, hipStream_t stream);
+
 // Largest batch of the fast decode kernel's balanced mode (its per-wave
 // prefix sums of blocks per sequence live in LDS).
 constexpr int kBalMaxB = 4096;

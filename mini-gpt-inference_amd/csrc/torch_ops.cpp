@@ -204,6 +204,79 @@ at::Tensor paged_prefill(const at::Tensor& q, const at::Tensor& kp, const at::Te
   return out;
 }
 
+// Whether t is a plain contiguous, 16-byte aligned tensor of x's dtype and
+// (current) device with `numel` elements: what the decode-step linear kernels
+// take.
+bool linear_ok(const at::Tensor& t, const at::Tensor& x, int64_t numel) {
+  return t.scalar_type() == x.scalar_type() && t.device() == x.device() && t.numel() == numel &&
+         t.device().index() == c10::hip::current_device() && t.layout() == at::kStrided && t.is_contiguous() &&
+         !t.is_neg() &&
+         (reinterpret_cast<uintptr_t>(t.data_ptr()) & 15u) == 0;
+}
+bool linear_ok(const c10::optional<at::Tensor>& t, const at::Tensor& x, int64_t numel) {
+  return !t || linear_ok(*t, x, numel);
+}
+void* ptr(const c10::optional<at::Tensor>& t) { return t ? t->data_ptr() : nullptr; }
+
+constexpr int64_t kLinearRows = 64;
+
+// decode_linear(x, weight, bias, gelu): act(x W^T + bias) for x [B, 1, K] -> [B, 1, N]; None when the call is not one the kernel takes
+// (the caller then makes the PyTorch calls it stands for).
+py::object decode_linear(const at::Tensor& x, const at::Tensor& w, const c10::optional<at::Tensor>& bias,
+                         bool gelu) {
+  if (!x.is_cuda() || x.dim() != 3 || x.size(1) != 1 || w.dim() != 2) return py::none();
+  const int64_t B = x.size(0), K = x.size(2), N = w.size(0);
+  const int dt = dtype_code(x.scalar_type());
+  if ((dt != MGI_BF16 && dt != MGI_F16) || B < 1 || B > kLinearRows || K < 64 || K % 64 != 0 || K > 2560 || N < 1 ||
+      w.size(1) != K || (B > 48 && K > 1536 && !gelu))
+    return py::none();
+  if (!linear_ok(x, x, B * K) || !linear_ok(w, x, N * K) || !linear_ok(bias, x, N))
+    return py::none();
+  at::Tensor out = at::empty({B, 1, N}, x.options());
+  check_status(mgi_decode_linear(out.data_ptr(), x.data_ptr(), w.data_ptr(), ptr(bias), gelu, dt, B, N, K,
+                                 stream_of(x)));
+  return py::cast(out);
+}
+
+// decode_linear_norm(x, weight, bias, residual, ln_weight, ln_bias, ln_eps) ->
+// (h, LN(h)) with h = x W^T + bias + residual, or (h, None) without the
+// LayerNorm pair; None when the call is not one the kernel takes. With x and
+// weight None: (residual, LN(residual)).
+py::object decode_linear_norm(const c10::optional<at::Tensor>& x, const c10::optional<at::Tensor>& w,
+                              const c10::optional<at::Tensor>& bias, const at::Tensor& residual,
+                              const c10::optional<at::Tensor>& ln_w, const c10::optional<at::Tensor>& ln_b,
+                              double ln_eps) {
+  const at::Tensor& r = residual;
+  if (!r.is_cuda() || r.dim() != 3 || r.size(1) != 1 || x.has_value() != w.has_value()) return py::none();
+  const int64_t B = r.size(0), N = r.size(2);
+  const int dt = dtype_code(r.scalar_type());
+  if ((dt != MGI_BF16 && dt != MGI_F16) || B < 1 || B > kLinearRows || N < 4 || N % 4 != 0 || N > 4096 ||
+      ln_w.has_value() != ln_b.has_value() || (!x && !ln_w))
+    return py::none();
+  int64_t K = 0;
+  if (x) {
+    if (x->dim() != 3 || x->size(0) != B || x->size(1) != 1 || w->dim() != 2) return py::none();
+    K = x->size(2);
+    if (K < 64 || K % 64 != 0 || w->size(0) != N || w->size(1) != K || !linear_ok(*x, r, B * K) ||
+        !linear_ok(*w, r, N * K))
+      return py::none();
+  }
+  if (!linear_ok(r, r, B * N) || !linear_ok(bias, r, N) || !linear_ok(ln_w, r, N) || !linear_ok(ln_b, r, N))
+    return py::none();
+  at::Tensor out, norm, ws;
+  size_t ws_bytes = 0;
+  if (x) {
+    out = at::empty({B, 1, N}, r.options());
+    ws_bytes = mgi_decode_linear_norm_workspace_bytes(B, N, K);
+    ws = at::empty({(int64_t)ws_bytes}, r.options().dtype(at::kByte));
+  }
+  if (ln_w) norm = at::empty({B, 1, N}, r.options());
+  check_status(mgi_decode_linear_norm(x ? out.data_ptr() : nullptr, ln_w ? norm.data_ptr() : nullptr, ptr(x), ptr(w),
+                                      ptr(bias), r.data_ptr(), ptr(ln_w), ptr(ln_b), (float)ln_eps, dt, B, N, K,
+                                      x ? ws.data_ptr() : nullptr, ws_bytes, stream_of(r)));
+  return py::make_tuple(x ? out : residual, ln_w ? py::cast(norm) : py::object(py::none()));
+}
+
 }  // namespace
 
 PYBIND11_MODULE(_hip_ops, m) {
@@ -212,4 +285,6 @@ PYBIND11_MODULE(_hip_ops, m) {
   m.def("paged_decode", &paged_decode);
   m.def("paged_decode_append", &paged_decode_append);
   m.def("paged_prefill", &paged_prefill);
+  m.def("decode_linear", &decode_linear);
+  m.def("decode_linear_norm", &decode_linear_norm);
 }

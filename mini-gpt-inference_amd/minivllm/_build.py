@@ -43,7 +43,7 @@ HIP_FLAGS = [
 # the prefill kernel's MFMA results in AGPRs and copies them back and forth
 # for the softmax (64 v_accvgpr moves per key tile).
 MFMA_FLAGS = ["-mllvm", "-amdgpu-mfma-vgpr-form"]
-MFMA_SOURCES = {"paged_prefill.hip"}
+MFMA_SOURCES = {"decode_linear.hip", "paged_prefill.hip"}
 
 
 def library_path() -> Path:

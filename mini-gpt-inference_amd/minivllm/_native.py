@@ -39,6 +39,9 @@ EXPORTED_SYMBOLS = (
     "mgi_paged_decode_balanced_waves",
     "mgi_paged_prefill",
     "mgi_paged_prefill_workspace_bytes",
+    "mgi_decode_linear",
+    "mgi_decode_linear_norm",
+    "mgi_decode_linear_norm_workspace_bytes",
 )
 
 _lock = threading.Lock()
@@ -112,6 +115,20 @@ def _declare(lib: ctypes.CDLL) -> None:
     ]
     lib.mgi_paged_prefill_workspace_bytes.restype = ctypes.c_size_t
     lib.mgi_paged_prefill_workspace_bytes.argtypes = [_i64, _i64, _i64, _i64, _i]
+    lib.mgi_decode_linear.restype = _i
+    lib.mgi_decode_linear.argtypes = [
+        _p, _p, _p, _p, _i, _i,            # out, x, weight, bias, gelu, dtype
+        _i64, _i64, _i64, _p,              # B N K, stream
+    ]
+    lib.mgi_decode_linear_norm.restype = _i
+    lib.mgi_decode_linear_norm.argtypes = [
+        _p, _p, _p, _p, _p, _p,            # out, norm, x, weight, bias, residual
+        _p, _p, ctypes.c_float, _i,        # LayerNorm weight, bias, eps; dtype
+        _i64, _i64, _i64,                  # B N K
+        _p, ctypes.c_size_t, _p,           # workspace, bytes, stream
+    ]
+    lib.mgi_decode_linear_norm_workspace_bytes.restype = ctypes.c_size_t
+    lib.mgi_decode_linear_norm_workspace_bytes.argtypes = [_i64, _i64, _i64]
 
 
 def lib() -> ctypes.CDLL:

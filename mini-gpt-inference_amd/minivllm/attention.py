@@ -40,6 +40,7 @@ import torch
 import torch.nn.functional as F
 from torch import Tensor, nn
 
+from . import decode_fused
 from .decode_batch_metadata import DecodeBatchMetadata
 from .kv_block_pool import KVBlockPool
 from .kv_runtime import KVRuntimeContext, PrefillChunkContext, PrefillRuntimeContext
@@ -227,7 +228,14 @@ class KVCacheCausalSelfAttention(nn.Module):
         B, T, C = x.shape
         assert T == 1
         q, k, v = self._qkv_heads(x)
-        q, k, v = q[:, 0], k[:, 0], v[:, 0]            # [B, H, D], row stride 3C
+        out = self._decode_attend(q[:, 0], k[:, 0], v[:, 0], metadata, kv_pool, layer_idx)
+        return self._finish(out)
+
+    def _decode_attend(self, q: Tensor, k: Tensor, v: Tensor, metadata: DecodeBatchMetadata, kv_pool: KVBlockPool,
+                       layer_idx: int) -> Tensor:
+        """KV append and paged attention of one decode step's q, k, v ([B, H, D],
+        row stride 3C) by the selected backend; [B, 1, C]."""
+        B = q.shape[0]
         backend = self.decode_attention_backend
         if backend == "reference":
             write_kv_rows(kv_pool, layer_idx, k, v, metadata.slot_mapping, use_hip=False)
@@ -252,7 +260,7 @@ class KVCacheCausalSelfAttention(nn.Module):
                                                     layer_idx=layer_idx)
         else:
             raise ValueError(f"unknown decode attention backend: {backend}")
-        return self._finish(out.reshape(B, 1, C))
+        return out.reshape(B, 1, self.n_embd)
 
     # -------------------------------------------------- dense (no paging)
 
@@ -276,3 +284,20 @@ class KVCacheCausalSelfAttention(nn.Module):
         att = self.attn_dropout(F.softmax(att, dim=-1))
         out = (att @ v.contiguous()).transpose(1, 2).reshape(B, T, C)
         return self._finish(out)
+
+
+_DECODE_METHODS = ("forward_decode_batch", "_qkv_heads", "_finish", "_decode_attend")
+_OWN_METHODS = tuple(KVCacheCausalSelfAttention.__dict__[n] for n in _DECODE_METHODS)
+
+
+def plain_decode_attention(attn: nn.Module) -> bool:
+    """Whether attn.forward_decode_batch is this module's own code over plain
+    projections, so its parts may be run one by one (decode_fused)."""
+    if type(attn) is not KVCacheCausalSelfAttention or not attn.__dict__.keys().isdisjoint(_DECODE_METHODS):
+        return False
+    cls = KVCacheCausalSelfAttention.__dict__
+    if tuple(cls.get(n) for n in _DECODE_METHODS) != _OWN_METHODS:
+        return False
+    m = attn._modules
+    return decode_fused.plain_linear(m["qkv"]) and decode_fused.plain_linear(m["project"]) \
+        and decode_fused.idle_dropout(m["resid_dropout"])

@@ -12,6 +12,7 @@ import torch.nn.functional as F
 from torch import Tensor, nn
 from torch.utils.checkpoint import checkpoint
 
+from . import decode_fused
 from .attention import DECODE_BACKENDS, PREFILL_MODES, KVCache
 from .block import TransformerBlock
 from .decode_batch_metadata import DecodeBatchMetadata
@@ -116,9 +117,33 @@ class MiniGPT(nn.Module):
     def decode_batch(self, input_ids: Tensor, metadata: DecodeBatchMetadata, kv_pool: KVBlockPool) -> Tensor:
         """One batched decode step: input_ids [B, 1] -> logits [B, 1, vocab]."""
         x = self._embed(input_ids, metadata.positions.unsqueeze(1))
-        for i, block in enumerate(self.blocks):
-            x = block.forward_decode_batch(x, metadata=metadata, kv_pool=kv_pool, layer_idx=i)
+        ops = decode_fused.ops_for(x)
+        width = x.shape[-1]
+        blocks = list(self.blocks)
+        plain = [ops is not None and type(b) is TransformerBlock and b._plain_decode(width) for b in blocks]
+        fused_head = self._plain_head(ops, width)
+        normed = None   # the next block's layer_norm_1(x), or the final layer_norm(x), when a fused call made it
+        for i, block in enumerate(blocks):
+            pair = None
+            if plain[i]:
+                last = i + 1 == len(blocks)
+                after = (self.layer_norm if fused_head else None) if last else \
+                    (blocks[i + 1].layer_norm_1 if plain[i + 1] else None)
+                pair = block._decode_step(ops, x, normed, after, metadata, kv_pool, i)
+            if pair is None:
+                x, normed = block.forward_decode_batch(x, metadata=metadata, kv_pool=kv_pool, layer_idx=i), None
+            else:
+                x, normed = pair
+        if fused_head and normed is not None:
+            head = self.language_model_head
+            logits = ops.decode_linear(normed, head.weight, head.bias, False)
+            return head(normed) if logits is None else logits
         return self._head(x)
+
+    def _plain_head(self, ops, width: int) -> bool:
+        """Whether _head is this class's own over plain modules (decode_fused)."""
+        return ops is not None and "_head" not in self.__dict__ and type(self)._head is _OWN_HEAD \
+            and decode_fused.plain_norm(self.layer_norm, width) and decode_fused.plain_linear(self.language_model_head)
 
     def decode(self, input_ids: Tensor, contexts: list[KVRuntimeContext]) -> Tensor:
         assert len(contexts) == self.n_layer
@@ -127,3 +152,6 @@ class MiniGPT(nn.Module):
         for i, block in enumerate(self.blocks):
             x = block.forward_decode(x, contexts[i])
         return self._head(x)
+
+
+_OWN_HEAD = MiniGPT._head
