@@ -249,6 +249,51 @@ int64_t split_partials(int64_t start, int64_t T, int64_t pk) {
   return n;
 }
 
+// Paged prefill key split of the fp32 kernel. Its workgroups run one 64-key
+// tile after another, tile_us each whether one or two share a CU, so a chunk
+// costs the longest of its chains or, where workgroups outnumber the CUs, a
+// CU's share of all tiles and half a chain; a workgroup adds about 2 us, the
+// split 8 us (merge launch, tail) and its partials written and read back at
+// 5 TB/s. The cheapest partition length is taken when it beats no split by a
+// tenth.
+// Measured on MI355X (us, without / with): 700 rows after 450, 8 heads, D = 64:
+// 67 / 30; 512 at 0: 32 / 16; 100 after 1000: 66 / 16; 256 after 4096, 16 heads,
+// D = 128: 513 / 183; 32 after 3000, 8 heads, D = 32: 122 / 14; 1024 after 1024,
+// 16 heads, D = 64: 138 / 96; 3000 at 0, 4 heads: 201 / 86. The split sums are
+// the closer ones to 64 bits (after 16 000 keys 4e-7 against 2.3e-6, the serial
+// sums' error growing by 1.4e-10 a key); chunks that end past kMaxSplitKeysF32
+// stay unsplit, so that no result moves by more than fp32 results are held to
+// (2.4e-6).
+constexpr int64_t kMaxSplitKeysF32 = 15360;
+int64_t prefill_split_keys_f32(int64_t start, int64_t T, int64_t H, int64_t D) {
+  const int dp = mgi::prefill_head_dim_bucket(0, (int)D);
+  if (D % 8 != 0 || dp == 0 || T <= 0 || start + T > kMaxSplitKeysF32) return 0;
+  const int64_t QB = T <= 32 ? 32 : 64, nq = (T + QB - 1) / QB;
+  auto tiles = [&](int64_t qt) { return (start + std::min(T, (qt + 1) * QB) + 63) / 64; };
+  if (nq * H >= 8 * (int64_t)device_cus()) return 0;  // rounds enough to even out
+  const double cus = (double)device_cus(), tile_us = dp == 32 ? 2.4 : dp == 64 ? 3.5 : 7.5;
+  int64_t total = 0;
+  for (int64_t qt = 0; qt < nq; ++qt) total += tiles(qt);
+  const double share = (double)(total * H) / cus;
+  auto cost = [&](int64_t k) {  // k tiles per partition
+    int64_t wgs = 0;
+    for (int64_t qt = 0; qt < nq; ++qt) wgs += (tiles(qt) + k - 1) / k;
+    return tile_us * std::max((double)k, share + 0.5 * (double)k) + 2.0 * (double)(wgs * H) / cus;
+  };
+  const int64_t longest = tiles(nq - 1);
+  double best_us = 0.9 * cost(longest);  // nearer than that, either may win
+  int64_t best = 0;
+  for (int64_t k = 1; k < longest; k += std::max<int64_t>(1, k / 8)) {
+    const double bytes = (double)split_partials(start, T, 64 * k) * (double)H * (double)(4 * D + 8);
+    const double us = cost(k) + 8.0 + 2.0 * bytes / 5.0e6;
+    if (us < best_us) {
+      best_us = us;
+      best = 64 * k;
+    }
+  }
+  return best;
+}
+
 // Paged prefill key split: keys per partition, or 0 for none. A chunk whose
 // workgroups (one per 64-row query tile and head, 32 rows for chunks of at
 // most 32) are fewer than two per CU leaves CUs idle and waits on its last
@@ -265,14 +310,15 @@ int64_t split_partials(int64_t start, int64_t T, int64_t pk) {
 // chunk at position 0: 18 -> 26 us split), so it needs a prefix at least as
 // long as the chunk: the model alone would split a 1024-row first chunk of
 // 16 heads, measured 28.9 -> 34.1 us (two workgroups per CU slow each tile
-// and the diagonal tiles take the masking path). 2-byte types with head_dim
-// a multiple of 8 only (the merge's lane layout).
+// and the diagonal tiles take the masking path). Head_dim a multiple of 8 only
+// (the merge's lane layout); fp32 has its own rule above.
 // MINIVLLM_HIP_PREFILL_SPLIT_KEYS = -1 turns it off; > 0 forces that many
-// keys per partition, rounded up to 64, without the cost model (tuning and
-// tests; read on every call).
+// keys per partition of the 2-byte types, rounded up to 64, without the cost
+// model (tuning and tests; read on every call).
 int64_t prefill_split_keys(int64_t start, int64_t T, int64_t H, int64_t D, int dtype) {
   const int forced = env_int("MINIVLLM_HIP_PREFILL_SPLIT_KEYS", 0);
-  if (forced < 0 || dtype == MGI_F32 || D % 8 != 0 || mgi::prefill_head_dim_bucket(1, (int)D) == 0 ||
+  if (dtype == MGI_F32) return forced == 0 ? prefill_split_keys_f32(start, T, H, D) : 0;
+  if (forced < 0 || D % 8 != 0 || mgi::prefill_head_dim_bucket(1, (int)D) == 0 ||
       T <= 0 || T > kMaxGridYZ)
     return 0;
   const int64_t QB = T <= 32 ? 32 : 64;
@@ -917,7 +963,9 @@ int mgi_paged_prefill(void* out, const int64_t* out_strides, const void* q,
     // bf16 chunk of 16 heads, as each thread then stages twice the tile.)
     a.cus = device_cus();
     const int waves = T <= 32 ? 2 : 4;
-    const PrefillWorkspace pw = prefill_workspace(start_pos, T, H, D, dtype);
+    PrefillWorkspace pw = prefill_workspace(start_pos, T, H, D, dtype);
+    if (dtype == MGI_F32 && (!workspace || workspace_bytes < pw.total || !aligned16(workspace)))
+      pw = PrefillWorkspace{};  // fp32 runs unsplit without a workspace, as it did before it had a split
     if (pw.part_keys > 0) {
       if (!workspace) return fail(MGI_EWORKSPACE, "workspace required for the split-key pass");
       if (workspace_bytes < pw.total)

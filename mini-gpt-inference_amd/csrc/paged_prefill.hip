@@ -136,6 +136,10 @@ template <> struct Mma16<float> {  // never called: fp32 takes the 16x16x4 path
   __device__ static __forceinline__ uint32_t pack2(float, float) { return 0u; }
 };
 
+__device__ __forceinline__ float f4_elem(const float4& x, int i) {
+  return i == 0 ? x.x : i == 1 ? x.y : i == 2 ? x.z : x.w;
+}
+
 // Column of key k (0..63) in a 2-byte V^T tile row. Keys 32c + 16h + 4g + i
 // sit at 32c + 8g + 4h + i, so the eight keys one lane feeds to a PV MFMA
 // (4g+i and 16+4g+i of a 32-key slice) are one 16-byte LDS read.
@@ -316,26 +320,35 @@ __global__ __launch_bounds__(64 * WAVES) void paged_prefill_mfma(const PrefillAr
     for (int b = 0; b < QPW; ++b)
 #pragma unroll
       for (int kb = 0; kb < 4; ++kb) s[b][kb] = f32x4_t{0.f, 0.f, 0.f, 0.f};
+    if constexpr (k16) {
 #pragma unroll
-    for (int kb = 0; kb < 4; ++kb) {
-      const T* krow = &kl[(16 * kb + col) * KROW];
+      for (int kb = 0; kb < 4; ++kb) {
+        const T* krow = &kl[(16 * kb + col) * KROW];
 #pragma unroll
-      for (int f = 0; f < NQF; ++f) {
-        if constexpr (k16) {
+        for (int f = 0; f < NQF; ++f) {
           const uint4 kv = *reinterpret_cast<const uint4*>(krow + 32 * f + 8 * g);
 #pragma unroll
           for (int b = 0; b < QPW; ++b) s[b][kb] = MM::mfma(kv, qf[b][f], s[b][kb]);
-        } else {
-          const float4 kv = *reinterpret_cast<const float4*>(krow + 16 * f + 4 * g);
-#pragma unroll
-          for (int b = 0; b < QPW; ++b) {
-            const float4 qv = __builtin_bit_cast(float4, qf[b][f]);
-            s[b][kb] = __builtin_amdgcn_mfma_f32_16x16x4f32(kv.x, qv.x, s[b][kb], 0, 0, 0);
-            s[b][kb] = __builtin_amdgcn_mfma_f32_16x16x4f32(kv.y, qv.y, s[b][kb], 0, 0, 0);
-            s[b][kb] = __builtin_amdgcn_mfma_f32_16x16x4f32(kv.z, qv.z, s[b][kb], 0, 0, 0);
-            s[b][kb] = __builtin_amdgcn_mfma_f32_16x16x4f32(kv.w, qv.w, s[b][kb], 0, 0, 0);
-          }
         }
+      }
+    } else {
+      // The four key blocks' products alternate, so no product waits for the
+      // one before it (each accumulator still sums in head-dim order).
+#pragma unroll
+      for (int f = 0; f < NQF; ++f) {
+        float4 kv[4];
+#pragma unroll
+        for (int kb = 0; kb < 4; ++kb)
+          kv[kb] = *reinterpret_cast<const float4*>(&kl[(16 * kb + col) * KROW] + 16 * f + 4 * g);
+#pragma unroll
+        for (int i = 0; i < 4; ++i)
+#pragma unroll
+          for (int b = 0; b < QPW; ++b)
+#pragma unroll
+            for (int kb = 0; kb < 4; ++kb)
+              s[b][kb] = __builtin_amdgcn_mfma_f32_16x16x4f32(f4_elem(kv[kb], i),
+                                                              f4_elem(__builtin_bit_cast(float4, qf[b][f]), i),
+                                                              s[b][kb], 0, 0, 0);
       }
     }
 
@@ -428,18 +441,19 @@ __global__ __launch_bounds__(64 * WAVES) void paged_prefill_mfma(const PrefillAr
       }
     } else {
 #pragma unroll
-      for (int kb = 0; kb < 4; ++kb)
+      for (int kb = 0; kb < 4; ++kb) {
+        float4 vv[NDB];
 #pragma unroll
-        for (int db = 0; db < NDB; ++db) {
-          const float4 vv = *reinterpret_cast<const float4*>(&vl[(16 * db + col) * VROW + 16 * kb + 4 * g]);
+        for (int db = 0; db < NDB; ++db)
+          vv[db] = *reinterpret_cast<const float4*>(&vl[(16 * db + col) * VROW + 16 * kb + 4 * g]);
 #pragma unroll
-          for (int b = 0; b < QPW; ++b) {
-            oacc[b][db] = __builtin_amdgcn_mfma_f32_16x16x4f32(vv.x, p[b][kb][0], oacc[b][db], 0, 0, 0);
-            oacc[b][db] = __builtin_amdgcn_mfma_f32_16x16x4f32(vv.y, p[b][kb][1], oacc[b][db], 0, 0, 0);
-            oacc[b][db] = __builtin_amdgcn_mfma_f32_16x16x4f32(vv.z, p[b][kb][2], oacc[b][db], 0, 0, 0);
-            oacc[b][db] = __builtin_amdgcn_mfma_f32_16x16x4f32(vv.w, p[b][kb][3], oacc[b][db], 0, 0, 0);
-          }
-        }
+        for (int i = 0; i < 4; ++i)
+#pragma unroll
+          for (int b = 0; b < QPW; ++b)
+#pragma unroll
+            for (int db = 0; db < NDB; ++db)
+              oacc[b][db] = __builtin_amdgcn_mfma_f32_16x16x4f32(f4_elem(vv[db], i), p[b][kb][i], oacc[b][db], 0, 0, 0);
+      }
     }
   };
 
