@@ -294,33 +294,94 @@ int64_t prefill_split_keys_f32(int64_t start, int64_t T, int64_t H, int64_t D) {
   return best;
 }
 
-// Paged prefill key split: keys per partition, or 0 for none. A chunk whose
-// workgroups (one per 64-row query tile and head, 32 rows for chunks of at
-// most 32) are fewer than two per CU leaves CUs idle and waits on its last
-// query tile, which folds every key tile of the prefix. Splitting each query
-// tile's keys into partitions of k tiles, k about the total key tiles over
-// two per CU (at least 2), spreads that work; the partials are combined by
-// paged_decode_merge. The split is taken when a cost model fitted on MI355X
-// (bf16, head_dim 128, 8-32 heads, chunks of 64-2048 rows after prefixes of
-// 0-16k tokens) says it pays: a lone workgroup takes ~1.5 us per 64-key
-// tile (scaled with head_dim), and the split adds ~8 us (merge launch, tail)
-// plus its fp32 partials written and read back at ~5 TB/s. It pays after
-// long prefixes (a 256-row chunk after 3000 tokens, 32 heads: 80 -> 41 us)
-// and not for chunks whose causal triangle is most of the work (a 512-row
-// chunk at position 0: 18 -> 26 us split), so it needs a prefix at least as
-// long as the chunk: the model alone would split a 1024-row first chunk of
-// 16 heads, measured 28.9 -> 34.1 us (two workgroups per CU slow each tile
-// and the diagonal tiles take the masking path). Head_dim a multiple of 8 only
-// (the merge's lane layout); fp32 has its own rule above.
+// Paged prefill key split of the 2-byte types: keys per partition (0: none) and
+// the kernel configuration for it (0: the launcher's choice).
+struct PrefillSplit {
+  int64_t keys;
+  int cfg;
+};
+
+// The cheapest split of a chunk of more than 32 rows on the direct-to-LDS
+// kernel, or none. Without one, the last query tile's chain of n key tiles
+// sets the time; with the keys of each query tile cut into partitions of k
+// tiles, a chunk takes k tiles per round of workgroups and a fixed 10-13 us
+// (launches, prologue, merge), and writes and reads its fp32 partials at 5
+// TB/s. The candidates fill the CUs once, twice or three times: 412 (64
+// rows, two workgroups per CU), 1422 (128 rows, one), 422 (128 rows, two),
+// with the us per tile measured at D = 128 and D = 64; the 412 and 1422
+// tiles cost more when H is no multiple of 8, as a head's workgroups then
+// spread over the XCDs. `plain`, the split with one partition length (total
+// tiles over two per CU), stays unless a candidate is 7 % cheaper: nearer
+// than that the estimates don't tell them apart. Measured on MI355X, plain
+// / this (us, bf16, D = 128): 300 rows after 15 000, 32 heads: 183 / 117;
+// 640 after 15 000: 226 / 186; 400 after 6000, 20 heads: 86 / 55; 900 after
+// 3000, 16 heads: 59 / 46; 450 after 5000, 32 heads: 66 / 58; 1100 after
+// 5000, 12 heads: 83 / 66; 500 after 10 000, 12 heads, D = 64: 47 / 37;
+// 1500 after 11 700, 12 heads: 190 / 158.
+PrefillSplit cheapest_prefill_split(int64_t start, int64_t T, int64_t H, int64_t D, const PrefillSplit& plain) {
+  struct Config {
+    int cfg, rows, per_cu;
+    double fixed_us, tile_us, sparse_us;  // per tile: full CUs; at most one workgroup per CU
+  };
+  const bool wide = D > 64, xcd = H % 8 == 0;
+  const Config configs[] = {
+      {412, 64, 2, 10.0, (wide ? 1.15 : 0.65) * (xcd ? 1.0 : 1.3), wide ? 0.95 : 0.6},
+      {1422, 128, 1, 13.0, (wide ? 1.07 : 0.65) * (xcd ? 1.0 : 1.15), (wide ? 1.07 : 0.65) * (xcd ? 1.0 : 1.15)},
+      {422, 128, 2, 12.0, wide ? 1.85 : 1.1, wide ? 1.4 : 0.9},
+  };
+  const int64_t cus = device_cus(), n = (start + T + 63) / 64, w64 = (T + 63) / 64 * H;
+  auto wgs_of = [&](const Config& c, int64_t k) {  // workgroups with partitions of k tiles
+    int64_t w = 0;
+    for (int64_t q0 = 0; q0 < T; q0 += c.rows) w += ((start + std::min(T, q0 + c.rows) + 63) / 64 + k - 1) / k;
+    return w * H;
+  };
+  auto cost = [&](const Config& c, int64_t k) {
+    const int64_t wgs = wgs_of(c, k);
+    const double r = (double)wgs / (double)(c.per_cu * cus), over = r - std::floor(r);
+    // A last round of a few workgroups starts as the shorter chains end.
+    const double rounds = r <= 1.0 ? 1.0 : over <= 0.07 ? r : std::ceil(r);
+    const double bytes = (double)split_partials(start, T, 64 * k) * (double)H * (double)(4 * D + 8);
+    return c.fixed_us + (double)k * rounds * (wgs <= cus ? c.sparse_us : c.tile_us) + 2.0 * bytes / 5.0e6;
+  };
+  PrefillSplit best = plain;
+  const double margin = 0.93;
+  double best_us = margin * (plain.keys > 0 ? cost(configs[plain.cfg == 412 ? 0 : 1], plain.keys / 64)
+                                            : 6.5 + (w64 > cus ? 1.6 : 1.0) * (wide ? 0.72 : 0.43) * (double)n);
+  for (const Config& c : configs) {
+    for (int64_t fill = 1; fill <= 3 * c.per_cu; ++fill) {
+      if (fill * cus < 2 * ((T + c.rows - 1) / c.rows) * H) continue;
+      // The shortest partitions whose workgroups fit: from the mean up.
+      int64_t k = std::max<int64_t>(2, wgs_of(c, 1) / (fill * cus));
+      while (k < n && wgs_of(c, k) > fill * cus) ++k;
+      if (k >= n || (n + k - 1) / k > kMaxGridYZ) continue;
+      const double us = cost(c, k);
+      if (us < best_us) {
+        best_us = us;
+        best = {64 * k, c.cfg};
+      }
+    }
+  }
+  return best;
+}
+
+// The key split of a call. Splitting pays after long prefixes (a 256-row chunk
+// after 3000 tokens, 32 heads: 80 -> 41 us) and not for chunks whose causal
+// triangle is most of the work (a 512-row chunk at position 0: 18 -> 26 us
+// split; 1024 rows, 16 heads: 28.9 -> 34.1), so it needs a prefix at least as
+// long as the chunk, and fewer than two 64-row workgroups (32 rows for chunks
+// of at most 32) per CU. The plain split, of the total key tiles over two per
+// CU (at least 2), is taken when a tile's 1.5 us (scaled with head_dim) saves
+// more than the split's 8 us and its partials cost; head dims with a
+// direct-to-LDS kernel then look for a cheaper one. Head_dim a multiple of 8 only (the merge's
+// lane layout); fp32 has its own rule above.
 // MINIVLLM_HIP_PREFILL_SPLIT_KEYS = -1 turns it off; > 0 forces that many
 // keys per partition of the 2-byte types, rounded up to 64, without the cost
-// model (tuning and tests; read on every call).
-int64_t prefill_split_keys(int64_t start, int64_t T, int64_t H, int64_t D, int dtype) {
+// models (tuning and tests; read on every call).
+PrefillSplit prefill_split(int64_t start, int64_t T, int64_t H, int64_t D, int dtype) {
   const int forced = env_int("MINIVLLM_HIP_PREFILL_SPLIT_KEYS", 0);
-  if (dtype == MGI_F32) return forced == 0 ? prefill_split_keys_f32(start, T, H, D) : 0;
-  if (forced < 0 || D % 8 != 0 || mgi::prefill_head_dim_bucket(1, (int)D) == 0 ||
-      T <= 0 || T > kMaxGridYZ)
-    return 0;
+  if (dtype == MGI_F32) return {forced == 0 ? prefill_split_keys_f32(start, T, H, D) : 0, 0};
+  const int dp = mgi::prefill_head_dim_bucket(1, (int)D);
+  if (forced < 0 || D % 8 != 0 || dp == 0 || T <= 0 || T > kMaxGridYZ) return {};
   const int64_t QB = T <= 32 ? 32 : 64;
   const int64_t nq = (T + QB - 1) / QB;
   int64_t total = 0, longest = 0;
@@ -331,27 +392,37 @@ int64_t prefill_split_keys(int64_t start, int64_t T, int64_t H, int64_t D, int d
   }
   if (forced > 0) {
     const int64_t pk = round_up(forced, 64);
-    return pk < longest * 64 && (start + T + pk - 1) / pk <= kMaxGridYZ ? pk : 0;  // partitions: grid y
+    return {pk < longest * 64 && (start + T + pk - 1) / pk <= kMaxGridYZ ? pk : 0, 0};  // partitions: grid y
   }
   const int64_t slots = 2 * (int64_t)device_cus();
-  if (nq * H >= slots || start < T) return 0;
+  if (nq * H >= slots || start < T) return {};
   const int64_t k = std::max<int64_t>(2, (total * H + slots - 1) / slots);
-  if (k >= longest) return 0;
-  const double tile_us = 1.5 * (double)std::max<int64_t>(D, 64) / 128.0;
-  const double partial_bytes = (double)split_partials(start, T, 64 * k) * (double)H * (double)(4 * D + 8);
-  const double split_us = (double)k * tile_us + 8.0 + 2.0 * partial_bytes / 5.0e6;
-  return split_us < (double)longest * tile_us && (start + T + 64 * k - 1) / (64 * k) <= kMaxGridYZ ? 64 * k : 0;
+  PrefillSplit plain{};
+  if (k < longest) {
+    const double tile_us = 1.5 * (double)std::max<int64_t>(D, 64) / 128.0;
+    const double partial_bytes = (double)split_partials(start, T, 64 * k) * (double)H * (double)(4 * D + 8);
+    const double split_us = (double)k * tile_us + 8.0 + 2.0 * partial_bytes / 5.0e6;
+    const int64_t parts = (start + T + 64 * k - 1) / (64 * k);
+    // Two groups per workgroup pay where their 128-row tiles fill the CUs and
+    // a partition is long.
+    if (split_us < (double)longest * tile_us && parts <= kMaxGridYZ)
+      plain = {64 * k, (T + 127) / 128 * H * parts >= device_cus() && k >= 32 ? 1422 : 412};
+  }
+  return T > 32 && (dp == 64 || dp == 128) ? cheapest_prefill_split(start, T, H, D, plain) : plain;
 }
 
 struct PrefillWorkspace {
   int64_t part_keys, max_parts;
+  int cfg;
   size_t ml_offset, total;
 };
 
 // [acc: T*H*max_parts*D f32 | ml: T*H*max_parts float2], 256-byte aligned.
 PrefillWorkspace prefill_workspace(int64_t start, int64_t T, int64_t H, int64_t D, int dtype) {
   PrefillWorkspace w{};
-  w.part_keys = prefill_split_keys(start, T, H, D, dtype);
+  const PrefillSplit split = prefill_split(start, T, H, D, dtype);
+  w.part_keys = split.keys;
+  w.cfg = split.cfg;
   if (w.part_keys == 0) return w;
   w.max_parts = (start + T + w.part_keys - 1) / w.part_keys;
   const int64_t n = T * H * w.max_parts;
@@ -973,6 +1044,7 @@ int mgi_paged_prefill(void* out, const int64_t* out_strides, const void* q,
       if (!aligned16(workspace)) return fail(MGI_EINVAL, "workspace must be 16-byte aligned");
       a.part_keys = (int)pw.part_keys;
       a.max_parts = (int)pw.max_parts;
+      a.split_cfg = pw.cfg;
       a.ws_acc = static_cast<float*>(workspace);
       a.ws_ml = reinterpret_cast<float2*>(static_cast<char*>(workspace) + pw.ml_offset);
     }

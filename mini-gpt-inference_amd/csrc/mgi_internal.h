@@ -98,6 +98,7 @@ struct PrefillArgs {
   int cus;            // compute units of the device (set by the caller)
   int part_keys;      // > 0: keys per partition (a multiple of 64) when the keys are split
   int max_parts;      // split keys: partitions per row the workspace holds
+  int split_cfg;      // split keys: paged_prefill_tr configuration (0: by partition length)
   float* ws_acc;      // split keys: [T, H, max_parts, D] unnormalised partial outputs
   float2* ws_ml;      // split keys: [T, H, max_parts] partial (max, sum), log2 domain
 };

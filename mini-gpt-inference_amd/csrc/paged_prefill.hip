@@ -1350,13 +1350,10 @@ int prefill_tr_mode() {
 //     14.5), and first chunks (start 0) whose 64-row tiles take up to two
 //     rounds of the CUs (1536 rows: 26.8 against 31.3 for 412; 8 heads,
 //     3072 rows: 40.5 against 54.1);
-//   * with the keys split over workgroups (the cost model sizes partitions
-//     for 64-row tiles): 1422 when its 128-row tiles times the partitions
-//     fill the CUs and a partition holds at least 32 key tiles (512 rows
-//     after 16 384: 83 against 98 us for 412; after 8192: 51.7 / 58.4; 32
-//     heads, 256 after 8192: 53 / 58), else 412 (256 after 4096: 27 against
-//     29 for 1422; 32 heads, 512 after 2048, 19-tile partitions: 45.6 /
-//     48.6), whose two-group hand-over does not pay on short partitions;
+//   * with the keys split over workgroups, what the split's cost model priced
+//     (412, 422 or 1422); for a forced partition length 1422 when its 128-row
+//     tiles times the partitions fill the CUs and a partition holds at least 32
+//     key tiles, else 412;
 //   * 412 (two workgroups of four 16-row wavefronts per CU) otherwise, and
 //     for chunks whose keys fit one tile (64 rows at 0, 16 and 32 heads:
 //     8.4-8.5 against 9.4-9.6 us for 1412).
@@ -1365,6 +1362,7 @@ int prefill_tr_choice(const PrefillArgs& a) {
   if (forced >= 0) return forced;
   const int64_t wgs128 = ((int64_t)a.T + 127) / 128 * a.H, wgs64 = ((int64_t)a.T + 63) / 64 * a.H;
   const int64_t wgs_paired = (((int64_t)a.T + 63) / 64 + 1) / 2 * a.H;
+  if (a.part_keys > 0 && a.split_cfg > 0) return a.split_cfg;
   if (a.part_keys > 0)
     return wgs128 * a.max_parts >= a.cus && a.part_keys >= 32 * kTileKeys ? 1422 : 412;
   if (a.start + a.T <= kTileKeys) return 412;  // one key tile: a second group would idle

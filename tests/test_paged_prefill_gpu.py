@@ -503,3 +503,27 @@ def test_strided_outputs(dtype):
                              start, layer)
     np.testing.assert_allclose(got, want, **TOL[dtype])
     assert torch.isnan(wide[..., D:]).all(), "the padding columns must stay untouched"
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16], ids=["bf16", "f16"])
+@pytest.mark.parametrize("start,T,H,D", [(15000, 300, 32, 128), (16000, 1000, 8, 128), (6000, 400, 20, 128),
+                                         (10000, 500, 12, 64), (8000, 64, 16, 128), (2000, 129, 3, 96), (1000, 33, 2, 56)])
+def test_priced_key_split_agrees_with_unsplit(monkeypatch, start, T, H, D, dtype):
+    """The configurations the split's cost model picks (64- and 128-row tiles,
+    one or two groups, one to several rounds), against the call unsplit: each
+    output is rounded once to dtype on both sides and each weight once, so the
+    rows differ by less than two of its half-ulps (2^-8, 2^-11) in norm."""
+    assert hpd._native.lib().mgi_paged_prefill_workspace_bytes(start, T, H, D, hpd._native.DTYPE_CODES[dtype]) > 0
+    g = torch.Generator(device=DEV).manual_seed(T)
+    n = -(-(start + T) // 16)
+    pool = KVBlockPool(1, n + 2, 16, H, D, device=DEV, dtype=dtype)
+    pool.k.normal_(generator=g)
+    pool.v.normal_(generator=g)
+    table = torch.randperm(n + 2, generator=torch.Generator().manual_seed(T))[:n]
+    q = torch.randn((T, H, D), generator=g, device=DEV).to(dtype)
+    out = run_hip(q, pool, table, start, 0).double()
+    monkeypatch.setenv("MINIVLLM_HIP_PREFILL_SPLIT_KEYS", "-1")
+    whole = run_hip(q, pool, table, start, 0).double()
+    err = ((out - whole).norm() / whole.norm()).item()
+    print(f"  split against unsplit: {err:.2e}", flush=True)
+    assert err <= (2.0 ** -8 if dtype == torch.bfloat16 else 2.0 ** -11)
