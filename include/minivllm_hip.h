@@ -264,8 +264,10 @@ int64_t mgi_paged_decode_balanced_waves(int64_t B, int64_t H, int64_t D,
  * when a cost model says it pays, split over several workgroups per query tile and the
  * partials merged in a second pass; workspace must then hold
  * mgi_paged_prefill_workspace_bytes(...) bytes for the same (start_pos, T,
- * H, D, dtype), and it may be NULL when that is 0, and in fp32, which then
- * runs unsplit. Its contents need no initialisation; calls that overlap in time need separate workspaces.
+ * H, D, dtype), and it may be NULL when that is 0. A workspace that is missing
+ * or smaller gets the plain split of the total key tiles over two workgroups
+ * per CU (2-byte types; MGI_EWORKSPACE when that one does not fit either), or
+ * no split. Its contents need no initialisation; calls that overlap in time need separate workspaces.
  * MINIVLLM_HIP_PREFILL_SPLIT_KEYS (read on every call, by both functions)
  * turns the split off (-1) or forces that many keys per partition (> 0; fp32
  * then runs unsplit).

@@ -376,10 +376,11 @@ PrefillSplit cheapest_prefill_split(int64_t start, int64_t T, int64_t H, int64_t
 // lane layout); fp32 has its own rule above.
 // MINIVLLM_HIP_PREFILL_SPLIT_KEYS = -1 turns it off; > 0 forces that many
 // keys per partition of the 2-byte types, rounded up to 64, without the cost
-// models (tuning and tests; read on every call).
-PrefillSplit prefill_split(int64_t start, int64_t T, int64_t H, int64_t D, int dtype) {
+// models (tuning and tests; read on every call). plain_only: the plain split
+// alone (none in fp32).
+PrefillSplit prefill_split(int64_t start, int64_t T, int64_t H, int64_t D, int dtype, bool plain_only) {
   const int forced = env_int("MINIVLLM_HIP_PREFILL_SPLIT_KEYS", 0);
-  if (dtype == MGI_F32) return {forced == 0 ? prefill_split_keys_f32(start, T, H, D) : 0, 0};
+  if (dtype == MGI_F32) return {forced == 0 && !plain_only ? prefill_split_keys_f32(start, T, H, D) : 0, 0};
   const int dp = mgi::prefill_head_dim_bucket(1, (int)D);
   if (forced < 0 || D % 8 != 0 || dp == 0 || T <= 0 || T > kMaxGridYZ) return {};
   const int64_t QB = T <= 32 ? 32 : 64;
@@ -408,7 +409,7 @@ PrefillSplit prefill_split(int64_t start, int64_t T, int64_t H, int64_t D, int d
     if (split_us < (double)longest * tile_us && parts <= kMaxGridYZ)
       plain = {64 * k, (T + 127) / 128 * H * parts >= device_cus() && k >= 32 ? 1422 : 412};
   }
-  return T > 32 && (dp == 64 || dp == 128) ? cheapest_prefill_split(start, T, H, D, plain) : plain;
+  return T > 32 && (dp == 64 || dp == 128) && !plain_only ? cheapest_prefill_split(start, T, H, D, plain) : plain;
 }
 
 struct PrefillWorkspace {
@@ -418,9 +419,9 @@ struct PrefillWorkspace {
 };
 
 // [acc: T*H*max_parts*D f32 | ml: T*H*max_parts float2], 256-byte aligned.
-PrefillWorkspace prefill_workspace(int64_t start, int64_t T, int64_t H, int64_t D, int dtype) {
+PrefillWorkspace prefill_workspace(int64_t start, int64_t T, int64_t H, int64_t D, int dtype, bool plain_only) {
   PrefillWorkspace w{};
-  const PrefillSplit split = prefill_split(start, T, H, D, dtype);
+  const PrefillSplit split = prefill_split(start, T, H, D, dtype, plain_only);
   w.part_keys = split.keys;
   w.cfg = split.cfg;
   if (w.part_keys == 0) return w;
@@ -494,7 +495,7 @@ int64_t mgi_paged_decode_balanced_waves(int64_t B, int64_t H, int64_t D, int64_t
 
 size_t mgi_paged_prefill_workspace_bytes(int64_t start_pos, int64_t T, int64_t H, int64_t D, int dtype) {
   if (start_pos < 0 || T <= 0 || H <= 0 || D <= 0 || !valid_dtype(dtype)) return 0;
-  return prefill_workspace(start_pos, T, H, D, dtype).total;
+  return prefill_workspace(start_pos, T, H, D, dtype, false).total;
 }
 
 size_t mgi_paged_decode_workspace_bytes(int64_t B, int64_t H, int64_t D, int64_t S, int64_t M,
@@ -1034,9 +1035,11 @@ int mgi_paged_prefill(void* out, const int64_t* out_strides, const void* q,
     // bf16 chunk of 16 heads, as each thread then stages twice the tile.)
     a.cus = device_cus();
     const int waves = T <= 32 ? 2 : 4;
-    PrefillWorkspace pw = prefill_workspace(start_pos, T, H, D, dtype);
-    if (dtype == MGI_F32 && (!workspace || workspace_bytes < pw.total || !aligned16(workspace)))
-      pw = PrefillWorkspace{};  // fp32 runs unsplit without a workspace, as it did before it had a split
+    // A caller without room for the priced split (one that sizes its workspace
+    // for the plain one, or gives none) gets the plain split, or none.
+    PrefillWorkspace pw = prefill_workspace(start_pos, T, H, D, dtype, false);
+    if (pw.part_keys > 0 && (!workspace || workspace_bytes < pw.total || !aligned16(workspace)))
+      pw = prefill_workspace(start_pos, T, H, D, dtype, true);
     if (pw.part_keys > 0) {
       if (!workspace) return fail(MGI_EWORKSPACE, "workspace required for the split-key pass");
       if (workspace_bytes < pw.total)

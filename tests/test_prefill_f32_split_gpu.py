@@ -81,3 +81,33 @@ def test_rule_on_the_host(monkeypatch):
         n = ws_bytes(start, T, H, D)
         parts = [p for p in range(2, 300) if -(-T * H * p * D * 4 // 256) * 256 + T * H * p * 8 == n]
         assert len(parts) == 1
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("start,T,H", [(3000, 900, 16), (15000, 300, 32)])
+def test_bf16_workspace_too_small_for_the_priced_split(start, T, H):
+    """A workspace that holds less than the priced split's partials: the call
+    falls back to the plain split or refuses, as it did before, and never writes
+    past what it was given."""
+    lib, D, S = _native.lib(), 128, 16
+    n = -(-(start + T) // S)
+    pool_k = torch.randn((1, n, S, H, D), device=DEV).to(torch.bfloat16)
+    q = torch.randn((T, H, D), device=DEV).to(torch.bfloat16)
+    table = torch.randperm(n, device=DEV)
+    need = int(lib.mgi_paged_prefill_workspace_bytes(start, T, H, D, _native.MGI_BF16))
+    assert need > 0
+    outs = []
+    for nbytes in (need, need - 256):
+        ws = torch.full((need,), 77, dtype=torch.uint8, device=DEV)
+        out = torch.empty_like(q)
+        rc = lib.mgi_paged_prefill(
+            out.data_ptr(), _native.strides(out), q.data_ptr(), _native.strides(q), pool_k.data_ptr(), pool_k.data_ptr(),
+            _native.strides(pool_k), _native.strides(pool_k), _native.MGI_BF16, table.data_ptr(), 1, _native.MGI_I64, n,
+            start, T, H, D, S, n, 1, 0, D ** -0.5, ws.data_ptr(), nbytes, torch.cuda.current_stream().cuda_stream)
+        torch.cuda.synchronize()
+        assert rc in (_native.MGI_OK, _native.MGI_EWORKSPACE) and (nbytes < need or rc == _native.MGI_OK)
+        assert (ws[nbytes:] == 77).all()
+        if rc == _native.MGI_OK:
+            outs.append(out.double())
+    if len(outs) == 2:
+        assert ((outs[0] - outs[1]).norm() / outs[0].norm()).item() <= 2.0 ** -8
