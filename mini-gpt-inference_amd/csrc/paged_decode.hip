@@ -732,6 +732,7 @@ paged_decode_wg(const DecodeArgs a) {
   constexpr int EB = (int)sizeof(T);
   constexpr int DMAX = 8 * LPH;
   __shared__ float st_m[NW], st_l[NW];
+  __shared__ bool st_seen[NW];
   __shared__ __align__(16) float st_o[NW][DMAX];
   const int lane = (int)threadIdx.x & 63;
   const int wv = __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6);
@@ -800,6 +801,7 @@ paged_decode_wg(const DecodeArgs a) {
   };
 
   float m = -INFINITY, l = 0.f, acc[8];
+  bool seen = false;  // whether this row has folded any token
 #pragma unroll
   for (int i = 0; i < 8; ++i) acc[i] = 0.f;
   auto consume = [&](const Step<T, GT>& st, int nv) {
@@ -813,7 +815,10 @@ paged_decode_wg(const DecodeArgs a) {
       mb = fmaxf(mb, s[t]);
     }
     const float mn = fmaxf(m, mb);
-    const float mr = (nv == 0 && mn == -INFINITY) ? 0.f : mn;  // a row that has folded nothing yet stays empty
+    // Nothing but masked tokens and scores of -inf so far: weights of 0, and an
+    // empty state, so a later finite score is not lost to -inf - -inf = NaN.
+    const float mr = mn == -INFINITY ? 0.f : mn;
+    seen = seen || nv > 0;
     const float alpha = fast_exp2(m - mr);
     float psum = 0.f;
 #pragma unroll
@@ -852,6 +857,7 @@ paged_decode_wg(const DecodeArgs a) {
   }
 
   // The rows of the wavefront, then the wavefronts.
+  const bool wave_seen = __builtin_amdgcn_ballot_w64(seen) != 0;
 #pragma unroll
   for (int x = LPH; x < 64; x *= 2) {
     const float mo = __shfl_xor(m, x, 64), lo = __shfl_xor(l, x, 64);
@@ -867,6 +873,7 @@ paged_decode_wg(const DecodeArgs a) {
     if (lane == 0) {
       st_m[wv] = m;
       st_l[wv] = l;
+      st_seen[wv] = wave_seen;
     }
     if (sub_ok) {
       *reinterpret_cast<float4*>(&st_o[wv][Layout<T>::elem(sub, a.D, 0)]) = make_float4(acc[0], acc[1], acc[2], acc[3]);
@@ -882,7 +889,13 @@ paged_decode_wg(const DecodeArgs a) {
     f[w] = st_m[w] == -INFINITY ? 0.f : fast_exp2(st_m[w] - M);
     L = fmaf(f[w], st_l[w], L);
   }
-  const float inv = L > 0.f ? 1.f / L : 0.f;
+  float inv = L > 0.f ? 1.f / L : 0.f;
+  if (M == -INFINITY) {  // tokens, and every score -inf: NaN, as softmax; no tokens: zeros
+    bool any = false;
+#pragma unroll
+    for (int w = 0; w < NW; ++w) any = any || st_seen[w];
+    if (any) inv = __builtin_nanf("");
+  }
   T* orow = reinterpret_cast<T*>(a.out) + (int64_t)b * a.o_sb + (int64_t)h * a.o_sh;
   for (int d = (int)threadIdx.x; d < a.D; d += 64 * NW) {
     float o = 0.f;

@@ -66,6 +66,29 @@ def test_matches_reference_at_step_edges(D, S, H, dtype, waves, monkeypatch):
 
 @pytest.mark.parametrize("waves", [4, 8])
 @pytest.mark.parametrize("dtype", DTYPES)
+def test_scores_of_minus_infinity(dtype, waves, monkeypatch):
+    """A score of -inf is a weight of 0 wherever it stands -- alone in the last
+    granule, filling the first one, a row's only one, or all but one token of the
+    context -- and a context of nothing else is NaN, as softmax has it."""
+    monkeypatch.setenv("MINIVLLM_HIP_DECODE_WG", str(waves))
+    ctx = [5, 17, 40, 40, 3, 300, 8]
+    print(f"  -inf scores {dtype} waves={waves}", flush=True)
+    q, pool, tables, lens, layer = _small_case(len(ctx), 3, 32, 16, ctx, dtype, seed=21)
+    q = q.abs() + 0.5
+    # the -inf tokens of each sequence: its last, its first granule, two granules, all but one, all, every second
+    # one, the first half
+    gone = [[4], range(4), range(8, 16), [i for i in range(40) if i != 23], range(3), range(0, 300, 2), range(4)]
+    for b, tokens in enumerate(gone):
+        for i in tokens:
+            pool.k[layer, tables[b, i // 16], i % 16, :, 7] = -float("inf")
+    got = hip(q, fx.pool_to_device(pool, DEV), tables, lens, layer)
+    want = reference(q, pool, tables, lens, layer)
+    assert np.isnan(want[4]).all() and np.isfinite(np.delete(want, 4, 0)).all()
+    np.testing.assert_allclose(got, want, atol=TOL[dtype], rtol=TOL[dtype])
+
+
+@pytest.mark.parametrize("waves", [4, 8])
+@pytest.mark.parametrize("dtype", DTYPES)
 @pytest.mark.parametrize("D", [32, 96, 128])
 def test_fused_append_matches_two_calls(D, dtype, waves, monkeypatch):
     """Same pools and outputs, bit for bit, as the append kernel followed by
