@@ -61,8 +61,8 @@ const char* mgi_last_error(void);
  * mgi_paged_decode_balanced_waves and the even split of split_tokens = 0;
  * 1.02 the prefill key split (mgi_paged_prefill's workspace arguments and
  * mgi_paged_prefill_workspace_bytes); 1.03 mgi_paged_decode_noalloc; 1.04
- * mgi_paged_decode_append. mgi_decode_linear and mgi_decode_linear_norm came
- * later without a change to the others. */
+ * mgi_paged_decode_append. mgi_decode_linear, mgi_decode_linear_norm and
+ * mgi_paged_decode_workgroup_waves came later without a change to the others. */
 int mgi_abi_version(void);
 
 /*
@@ -116,7 +116,7 @@ int mgi_kv_append(void* k_pool, void* v_pool,
  *
  * split_tokens: 0 lets the library split the work. Small calls give each
  * (sequence, head) to one workgroup, in one launch and without using the
- * workspace. Otherwise, when a table is wider
+ * workspace (mgi_paged_decode_workgroup_waves). Otherwise, when a table is wider
  * than one partition and B <= 4096, it splits evenly: the blocks of all
  * sequences, in sequence order, are cut into equal segments, one per
  * wavefront of a fixed count (mgi_paged_decode_balanced_waves), whatever the
@@ -232,13 +232,21 @@ int64_t mgi_paged_decode_split_tokens(int64_t B, int64_t H, int64_t D,
                                       int64_t split_tokens);
 
 /* Wavefronts per group of heads of the even split for these sizes on the
- * current device (what mgi_paged_decode uses unless the call is small enough
- * for one workgroup per (sequence, head)), or 0 when it splits into
+ * current device (what mgi_paged_decode uses unless
+ * mgi_paged_decode_workgroup_waves is not 0), or 0 when it splits into
  * partitions (or does not split). No counterpart in the reference: it reports the
  * split, as mgi_paged_decode_split_tokens does. */
 int64_t mgi_paged_decode_balanced_waves(int64_t B, int64_t H, int64_t D,
                                         int64_t S, int64_t M,
                                         int64_t split_tokens);
+
+/* Wavefronts per workgroup when mgi_paged_decode gives each (sequence, head)
+ * of these sizes to one workgroup on the current device (q and the pool as the
+ * fast path wants them), or 0 when it takes the split the two functions above
+ * report. No counterpart in the reference. */
+int64_t mgi_paged_decode_workgroup_waves(int64_t B, int64_t H, int64_t D,
+                                         int64_t S, int64_t M, int dtype,
+                                         int64_t split_tokens);
 
 /*
  * Paged prefill attention of one chunk of one sequence.

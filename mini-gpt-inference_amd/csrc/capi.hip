@@ -152,42 +152,80 @@ SplitPlan split_plan(int64_t B, int64_t H, int64_t D, int64_t S, int64_t M, int6
 
 // Wavefronts per workgroup of the workgroup kernel (paged_decode_wg: one
 // workgroup per (sequence, head), one launch), or 0 to use the split chosen
-// above. It saves the context scan, the partials and the merge launch,
-// about 8 us; it loses where one workgroup's context is long (a CU alone
-// streams about 46 KB/us, and the longest context ends the call), on large
-// calls (its one-head pieces stream at 6.2 TB/s against 6.7, 64-byte ones
-// at 3.5) and where launching many short workgroups costs more than their
-// work (about 1.2 ns per wavefront). Balanced groups of 64 / LPH heads that
-// H does not fill stream at 1.25 times the filled share, at most all, of
-// their rate. Calls whose table fits one partition had one wavefront walk
-// each context alone, 0.14 us per token (0.18 in f32). The terms below are
-// those costs in us, for contexts that fill the table. Measured on MI355X
-// (us, without / with; bf16, D = 128 unless noted): 4 sequences x 8 heads,
-// D = 32, contexts 200-256, f32: 48 / 6.4; 13 x 16, 100-1000: 25.2 / 18.9;
-// 16 x 16, 256-768: 26.2 / 17.1; 32 x 8, 128-1024: 27.6 / 19.7; 128 x 16, D
-// = 64, 64-512: 37.0 / 34.3; 20 x 16, D = 96, 200-250: 42.8 / 11.7; 190 x
-// 4, D = 64, 4861-9723: 345 / 259; 139 x 2, 5262: 190 / 166. Kept on the
-// splits: 1 x 32 at 2000: 20.4 / 26.8; 4 x 32 at 4000: 52.7 / 56.1; 64 x 4,
-// 512-4096: 58.0 / 62.0; 256 x 32, 128-2048: 730 / 765; 256 x 16, D = 64,
-// 10-100: 14.7 / 21.6; 49 x 30, D = 32, 4642: 147 / 254; 53 x 2, D = 96,
-// 8085, f32: 175 / 199. Eight wavefronts, except four where a context is at
-// most half a step of the eight, or two steps on a large grid (22 x 22,
-// 29-59: 6.7 against 7.7; 200 x 8, D = 64, 16-512: 27.2 against 29.8).
+// above. Only the table's width M*S is known here, not the contexts in it, so
+// the kernel is taken where the split is not faster whichever rows are long:
+// one row that fills the table among short ones (the workgroups of that row,
+// one per head, end the call), half of the rows (the long workgroups share CUs
+// unevenly, 1.35 times the mean) and all of them. In us:
+//   workgroups  4.2 and the largest of 0.95 ns per wavefront launched; a long
+//               row's K and V per CU and round of the CUs, 23.5 us/MB (30 at 128
+//               bytes per head row, 40 where the row is no whole number of
+//               128-byte lines, 34-58 by H at head_dim up to 32; 1.6 times with
+//               four wavefronts); and all K and V at 6.2 TB/s (5.4, 3.8; 2.8
+//               and, in f32, 4.0)
+//   split       12 and all K and V at 6.7 TB/s, or 1.25 times the filled share
+//               of the lanes of its head groups if that is less; at least 18.5,
+//               or 22 for a few long rows among 8 or more (20 and 26 where heads
+//               fill at most half a group or head_dim not its lanes)
+//   one part    (the table fits one partition, one wavefront walks each
+//               context) 5.2 and 0.11 us per token of the longest, 0.18 in
+//               f32, or all K and V at 6.7 TB/s; up to 16 wavefronts per CU,
+//               with the longest context half of the table: the widths the
+//               runner pads tables to are within that
+// Measured on MI355X over 1725 shapes (1-256 sequences, 2-32 heads, head_dim
+// 32-256, tables of 32-8192 tokens), each with all rows full, random, one and
+// two full, half full and all short: where this takes the kernel, the split is
+// at most 8 % faster on any of the mixes with a context of half the table (5
+// shapes more than 5 %). Split / workgroups, us, bf16, D = 128: 13 x 16 heads,
+// 1024 tokens, one row full 24.4 / 16.4, all 29.4 / 21.5; 1 x 32, 1024: 19.0 /
+// 15.4; 32 x 16, 256, one partition: 29.2 / 14.5, all contexts 16 tokens: 5.3 /
+// 5.8 (64 x 16: 29.4 / 24.9, and 5.5 / 7.4); D = 32, f32, 4 x 8, 256: 48 / 5.7.
+// Left to the split: 13 x 16, 2048, one row full 24.8 / 28.0; 32 x 32, 1024,
+// half 54.0 / 54.0 and 64 x 16 61.3 / 54.4; D = 64, 64 x 4, 8192, one row full
+// 29.0 / 52.4, all 141 / 103; D = 32, 32 x 4, f32, 8192, one 33.4 / 87.7.
+// Eight wavefronts; four where a context is at most half a step of the eight
+// and where eight would be more than 8 per CU (one partition) or 32 (22 x 22,
+// 29-59: 6.7 against 7.7; 64 x 16, D = 64, one row of 512 full: 9.8 against 12.8).
 // MINIVLLM_HIP_DECODE_WG = 0 turns the kernel off, 4 or 8 forces it (tuning
 // and tests; read on every call).
 int wg_waves_for(int64_t B, int64_t H, int64_t D, int64_t S, int64_t M, int64_t eb, bool split) {
   const int forced = env_int("MINIVLLM_HIP_DECODE_WG", -1);
   if (forced >= 0) return forced == 0 ? 0 : forced == 4 ? 4 : 8;
   const int64_t lph = D <= 32 ? 4 : D <= 64 ? 8 : D <= 128 ? 16 : 32, hpw = 64 / lph;
+  const int64_t tokens = M * S, cus = device_cus(), line = D * eb;
   const int64_t step_tokens = 8 * hpw * (mgi::kGranuleLoads * 2 / eb);  // one step of eight wavefronts
-  const bool large_grid = B * H >= 4 * (int64_t)device_cus();
-  const int waves = M * S <= (large_grid ? 2 * step_tokens : step_tokens / 2) ? 4 : 8;
-  const double wg_mb = 2e-6 * (double)(M * S) * (double)(D * eb), all_mb = wg_mb * (double)(B * H);
-  const double filled = (double)H / (double)((H + hpw - 1) / hpw * hpw);  // of the balanced split's lanes
-  const double wg_us = std::max(all_mb / (D <= 32 ? 3.5 : 6.2), 1.2e-3 * (double)(B * H * waves)) + wg_mb * 10.9;
-  const double other_us = split ? 8.0 + all_mb / (6.7 * std::min(1.0, 1.25 * filled))
-                                : std::max(all_mb / 6.7, (eb == 4 ? 0.18 : 0.14) * (double)(M * S));
-  return wg_us < other_us ? waves : 0;
+  const int waves = tokens <= step_tokens / 2 || B * H * 8 > (split ? 32 : 8) * cus ? 4 : 8;
+  const double row_mb = 2e-6 * (double)tokens * (double)line;  // K and V of one full context and head
+  const double launch_us = 0.95e-3 * (double)(B * H * waves);
+  double us_per_mb = 23.5, tbps = 6.2;
+  if (D <= 32) {
+    us_per_mb = 34.0 + 1.5 * (double)std::min<int64_t>(H, 16);
+    tbps = eb == 2 ? 2.8 : 4.0;
+  } else if (line % 128 != 0) {
+    us_per_mb = 40.0;
+    tbps = 3.8;
+  } else if (line == 128) {
+    us_per_mb = 30.0;
+    tbps = 5.4;
+  }
+  if (!split) {
+    const double token_us = eb == 4 ? 0.18 : 0.11, all_mb = row_mb * (double)(B * H);
+    const bool pays = B * H * waves <= 16 * cus && 4.2 + launch_us <= 5.2 + 0.5 * token_us * (double)tokens &&
+                      4.2 + all_mb / tbps <= std::max(5.2 + token_us * (double)tokens, 3.0 + all_mb / 6.7);
+    return pays ? waves : 0;
+  }
+  const double long_us = row_mb * us_per_mb * (waves == 8 ? 1.0 : 1.6);
+  const double lanes = (double)((H + hpw - 1) / hpw * hpw);
+  const double split_tbps = 6.7 * std::min(1.0, 1.25 * (double)(H * D) / (lanes * 8.0 * (double)lph));
+  const bool sparse = 2.0 * (double)H <= lanes || D < 8 * lph;
+  auto pays = [&](double rows, double spread, double split_floor) {  // `rows` full contexts, the others short
+    const double mb = row_mb * rows * (double)H;
+    const double wg_us =
+        4.2 + std::max({std::ceil(rows * (double)H / (double)cus) * long_us, launch_us, spread * mb / tbps});
+    return wg_us <= std::max(split_floor, 12.0 + mb / split_tbps);
+  };
+  const double floor_us = sparse ? 20.0 : 18.5, few_us = B < 8 ? floor_us : sparse ? 26.0 : 22.0;
+  return pays(1.0, 1.0, few_us) && pays(0.5 * (double)B, 1.35, floor_us) && pays((double)B, 1.0, floor_us) ? waves : 0;
 }
 
 struct WorkspaceLayout {
@@ -491,6 +529,13 @@ int64_t mgi_paged_decode_balanced_waves(int64_t B, int64_t H, int64_t D, int64_t
                                         int64_t split_tokens) {
   if (B <= 0 || H <= 0 || D <= 0 || S <= 0 || M <= 0) return 0;
   return split_plan(B, H, D, S, M, split_tokens).bal_waves;
+}
+
+int64_t mgi_paged_decode_workgroup_waves(int64_t B, int64_t H, int64_t D, int64_t S, int64_t M, int dtype,
+                                         int64_t split_tokens) {
+  if (B <= 0 || H <= 0 || D <= 0 || S <= 0 || M <= 0 || !valid_dtype(dtype)) return 0;
+  if (split_tokens > 0 || D % 8 != 0 || D > 256 || S % (dtype == MGI_F32 ? 4 : 8) != 0) return 0;
+  return wg_waves_for(B, H, D, S, M, dtype_bytes(dtype), split_plan(B, H, D, S, M, split_tokens).max_parts > 1);
 }
 
 size_t mgi_paged_prefill_workspace_bytes(int64_t start_pos, int64_t T, int64_t H, int64_t D, int dtype) {

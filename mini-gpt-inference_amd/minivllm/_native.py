@@ -37,6 +37,7 @@ EXPORTED_SYMBOLS = (
     "mgi_paged_decode_workspace_bytes",
     "mgi_paged_decode_split_tokens",
     "mgi_paged_decode_balanced_waves",
+    "mgi_paged_decode_workgroup_waves",
     "mgi_paged_prefill",
     "mgi_paged_prefill_workspace_bytes",
     "mgi_decode_linear",
@@ -113,6 +114,8 @@ def _declare(lib: ctypes.CDLL) -> None:
         _p, ctypes.c_size_t,               # workspace, bytes
         _p,                                # stream
     ]
+    lib.mgi_paged_decode_workgroup_waves.restype = _i64
+    lib.mgi_paged_decode_workgroup_waves.argtypes = [_i64, _i64, _i64, _i64, _i64, _i, _i64]
     lib.mgi_paged_prefill_workspace_bytes.restype = ctypes.c_size_t
     lib.mgi_paged_prefill_workspace_bytes.argtypes = [_i64, _i64, _i64, _i64, _i]
     lib.mgi_decode_linear.restype = _i

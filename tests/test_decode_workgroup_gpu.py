@@ -12,6 +12,7 @@ import pytest
 import torch
 
 import _fixtures as fx
+from minivllm import _native
 from minivllm import hip_paged_decode as hpd
 from test_decode_append_gpu import bits, step_case
 from test_paged_decode_gpu import _small_case, hip
@@ -116,3 +117,19 @@ def test_split_kernels_still_match_where_the_rule_leaves_them(dtype, monkeypatch
     got = hip(q, fx.pool_to_device(pool, DEV), tables, lens, layer)
     want = reference(q, pool, tables, lens, layer)
     np.testing.assert_allclose(got, want, atol=TOL[dtype], rtol=TOL[dtype])
+
+
+@pytest.mark.parametrize("B,H,D,width,want", [(4, 8, 32, 16, 8), (22, 22, 128, 4, 4), (8, 4, 128, 128, 0)])
+def test_query_names_the_route_a_call_takes(B, H, D, width, want, monkeypatch):
+    """The call's bits are those of the route mgi_paged_decode_workgroup_waves
+    reports, and not those of the others: a table with one full row."""
+    monkeypatch.delenv("MINIVLLM_HIP_DECODE_WG", raising=False)
+    assert hpd._native.lib().mgi_paged_decode_workgroup_waves(B, H, D, 16, width, _native.MGI_F32, 0) == want
+    ctx = [16 * width] + [1 + (7 * b) % min(48, 16 * width) for b in range(1, B)]
+    q, pool, tables, lens, layer = _small_case(B, H, D, 16, ctx, torch.float32, seed=B)
+    pool, auto = fx.pool_to_device(pool, DEV), {}
+    auto["call"] = hip(q, pool, tables, lens, layer)
+    for w in (0, 4, 8):
+        monkeypatch.setenv("MINIVLLM_HIP_DECODE_WG", str(w))
+        auto[w] = hip(q, pool, tables, lens, layer)
+    assert [w for w in (0, 4, 8) if np.array_equal(auto[w], auto["call"])] == [want]
