@@ -24,6 +24,10 @@ class TransformerBlock(nn.Module):
         self.layer_norm_1 = nn.LayerNorm(n_embd)
         self.layer_norm_2 = nn.LayerNorm(n_embd)
 
+    # False: decode steps make the PyTorch calls for this block's norms, projections and MLP (and, on a model's last
+    # block, for the final norm and the LM head), whatever the attention backend.
+    fused_decode_linears = True
+
     def _mlp(self, x: Tensor) -> Tensor:
         return x + self.ffn(self.layer_norm_2(x))
 
@@ -51,7 +55,7 @@ class TransformerBlock(nn.Module):
         """Whether forward_decode_batch is this module's own code over plain
         submodules (decode_fused)."""
         m = self._modules
-        if type(self) is not TransformerBlock or not self.__dict__.keys().isdisjoint(_DECODE_METHODS) \
+        if not self.fused_decode_linears or type(self) is not TransformerBlock or not self.__dict__.keys().isdisjoint(_DECODE_METHODS) \
                 or tuple(TransformerBlock.__dict__.get(n) for n in _DECODE_METHODS) != _OWN_METHODS \
                 or not plain_decode_attention(m["attn"]) or m["attn"].n_embd != width:
             return False

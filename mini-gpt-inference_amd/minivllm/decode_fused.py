@@ -14,7 +14,9 @@ Whether a call may take this route is decided on every call from the tensors
 (in the binding, which returns None for what the kernels do not take) and the
 modules: only the plain module classes, without hooks, replaced methods,
 active dropout, autocast, gradients, tracing or transforms. Everything else
-makes the PyTorch calls. The choice does not depend on the attention backend.
+makes the PyTorch calls, and so does a block whose ``fused_decode_linears`` is
+False. The choice does not depend on the attention backend, so that switching
+the backend changes the attention alone.
 """
 from __future__ import annotations
 

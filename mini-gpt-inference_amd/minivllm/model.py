@@ -61,7 +61,10 @@ class MiniGPT(nn.Module):
         """'reference' (PyTorch) or 'hip' (MI355X kernels; 'triton_v0' is an alias).
 
         Constraints of the HIP backend (GPU tensors, supported dtypes) are
-        validated at dispatch and never bypassed.
+        validated at dispatch and never bypassed. The name selects the KV
+        append and the attention alone: a decode step's norms and linear
+        layers go through decode_fused under either (so the two differ in
+        attention only) unless a block's ``fused_decode_linears`` is False.
         """
         if backend not in DECODE_BACKENDS:
             raise ValueError("decode backend must be reference, hip or triton_v0")

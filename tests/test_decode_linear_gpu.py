@@ -195,6 +195,19 @@ def test_modules_and_contexts_that_keep_the_pytorch_calls(monkeypatch):
     with monkeypatch.context() as mp:
         mp.setattr(TransformerBlock, "_mlp", lambda self, x: x)
         assert fused_calls() == 0
+    for blk in model.blocks:
+        blk.fused_decode_linears = False
+    assert fused_calls() == 0
+    with torch.inference_mode():
+        off, _ = run()
+        monkeypatch.setattr(decode_fused, "ops_for", lambda x: None)
+        plain, _ = run()
+    assert torch.equal(off, plain)
+    monkeypatch.undo()
+    monkeypatch.setattr(_native, "ops", lambda: Spy())
+    for blk in model.blocks:
+        blk.fused_decode_linears = True
+    assert fused_calls() == full
     b.ffn.network[1].approximate = "tanh"
     assert fused_calls() < full
     b.ffn.network[1].approximate = "none"
