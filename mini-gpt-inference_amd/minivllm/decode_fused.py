@@ -12,20 +12,23 @@ calls; the bits differ.
 
 Whether a call may take this route is decided on every call from the tensors
 (in the binding, which returns None for what the kernels do not take) and the
-modules: only the plain module classes, without hooks, replaced methods,
-active dropout, autocast, gradients, tracing or transforms. Everything else
-makes the PyTorch calls, and so does a block whose ``fused_decode_linears`` is
-False. The choice does not depend on the attention backend, so that switching
-the backend changes the attention alone.
+modules: only the plain module classes, without hooks, replaced methods (the
+module's, its class's or the torch functions' they end in), active dropout,
+autocast, gradients, tracing or transforms. Everything else makes the PyTorch
+calls, and so does a block whose ``fused_decode_linears`` is False. The choice
+does not depend on the attention backend, so that switching the backend changes
+the attention alone.
 """
 from __future__ import annotations
 
 import torch
+import torch.nn.functional as F
 from torch import Tensor, nn
 from torch.autograd import forward_ad
 from torch.nn.modules import module as _nn_module
 
 from . import _native
+from .feed_forward import FeedForward
 
 MAX_ROWS = 64
 _DTYPES = (torch.bfloat16, torch.float16)
@@ -40,7 +43,7 @@ def ops_for(x: Tensor):
             or torch.compiler.is_compiling() or forward_ad._current_level >= 0 \
             or torch._C._len_torch_dispatch_stack() or torch._C._len_torch_function_stack() \
             or torch._C._functorch.peek_interpreter_stack() is not None \
-            or _nn_module._global_forward_hooks or _nn_module._global_forward_pre_hooks:
+            or _nn_module._global_forward_hooks or _nn_module._global_forward_pre_hooks or not unpatched():
         return None
     try:
         ops = _native.ops()
@@ -50,23 +53,40 @@ def ops_for(x: Tensor):
 
 
 def plain(m: nn.Module, cls: type) -> bool:
-    """Whether calling m runs cls.forward and nothing else."""
-    return type(m) is cls and not m._forward_hooks and not m._forward_pre_hooks and "forward" not in m.__dict__
+    """Whether calling m runs cls's own forward and nothing else."""
+    return type(m) is cls and cls.forward is _FORWARD[cls] and cls.__call__ is _CALL and not m._forward_hooks \
+        and not m._forward_pre_hooks and "forward" not in m.__dict__
+
+
+def unpatched() -> bool:
+    """Whether the functions those forwards end in are the ones this module was
+    imported with."""
+    return nn.Module._call_impl is _CALL_IMPL and all(getattr(F, n) is f for n, f in _FUNCTIONS.items())
+
+
+def plain_params(m: nn.Module, bias: tuple) -> bool:
+    """Whether m.weight and m.bias are m's own parameters (of one of the types
+    ``bias`` for the bias), not attributes or buffers put in their place."""
+    p = m._parameters
+    return type(p.get("weight")) is nn.Parameter and "bias" in p and type(p["bias"]) in bias \
+        and m.__dict__.keys().isdisjoint(_NAMES)
 
 
 def plain_linear(m: nn.Module) -> bool:
-    p = m._parameters
-    return plain(m, nn.Linear) and type(p.get("weight")) is nn.Parameter and type(p.get("bias")) in _PARAMS
+    return plain(m, nn.Linear) and plain_params(m, (nn.Parameter, type(None)))
 
 
 def plain_norm(m: nn.Module, width: int) -> bool:
-    p = m._parameters
-    return plain(m, nn.LayerNorm) and m.normalized_shape == (width,) and type(p.get("weight")) is nn.Parameter \
-        and type(p.get("bias")) is nn.Parameter
+    return plain(m, nn.LayerNorm) and m.normalized_shape == (width,) and plain_params(m, (nn.Parameter,))
 
 
 def idle_dropout(m: nn.Module) -> bool:
     return plain(m, nn.Dropout) and not (m.training and m.p > 0.0)
 
 
-_PARAMS = (nn.Parameter, type(None))
+_NAMES = ("weight", "bias")
+_CALL, _CALL_IMPL = nn.Module.__call__, nn.Module._call_impl
+# A forward from elsewhere than its class's module was patched before this import: nothing equals None.
+_FORWARD = {cls: cls.forward if cls.forward.__module__ == cls.__module__ else None
+            for cls in (nn.Linear, nn.LayerNorm, nn.GELU, nn.Dropout, nn.Sequential, FeedForward)}
+_FUNCTIONS = {n: getattr(F, n) for n in ("linear", "layer_norm", "gelu", "dropout")}

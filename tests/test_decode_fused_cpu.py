@@ -4,8 +4,13 @@ without a GPU."""
 from __future__ import annotations
 
 import pytest
+import torch
+import torch.nn.functional as F
+from torch import nn
 
+from minivllm import decode_fused
 from minivllm.block import TransformerBlock
+from minivllm.feed_forward import FeedForward
 from minivllm.model import MiniGPT
 
 
@@ -28,3 +33,55 @@ def test_the_attention_backend_does_not_choose(backend):
     model.set_decode_attention_backend(backend)
     assert all(b._plain_decode(64) for b in model.blocks)
     assert not any("fused_decode" in k for k in model.state_dict())
+
+
+@pytest.mark.parametrize("cls", [nn.Linear, nn.LayerNorm, nn.GELU, nn.Dropout, nn.Sequential, FeedForward])
+def test_a_replaced_class_method_is_called(block, cls, monkeypatch):
+    """A forward replaced on the class (as quantisers and profilers do) runs in
+    a decode step; so does a replaced __call__."""
+    forward = cls.forward
+    monkeypatch.setattr(cls, "forward", lambda self, *a, **kw: forward(self, *a, **kw))
+    assert not block._plain_decode(64)
+    monkeypatch.undo()
+    assert block._plain_decode(64)
+    monkeypatch.setattr(cls, "__call__", lambda self, *a, **kw: forward(self, *a, **kw), raising=False)
+    assert not block._plain_decode(64)
+    monkeypatch.undo()
+    assert block._plain_decode(64)
+
+
+@pytest.mark.parametrize("name", ["linear", "layer_norm", "gelu", "dropout"])
+def test_a_replaced_torch_function_is_called(name, monkeypatch):
+    assert decode_fused.unpatched()
+    function = getattr(F, name)
+    monkeypatch.setattr(F, name, lambda *a, **kw: function(*a, **kw))
+    assert not decode_fused.unpatched()
+    monkeypatch.undo()
+    monkeypatch.setattr(nn.Module, "_call_impl", lambda self, *a, **kw: self.forward(*a, **kw))
+    assert not decode_fused.unpatched()
+
+
+@pytest.mark.parametrize("path", ["attn.project", "ffn.network.0", "ffn.network.2", "layer_norm_1", "layer_norm_2"])
+@pytest.mark.parametrize("name", ["weight", "bias"])
+def test_attributes_in_place_of_parameters_are_used(block, path, name):
+    """A weight or bias taken out of the parameters and set as a plain tensor
+    (or put over the parameter in the module's dict) is what the module's
+    forward reads; a bias so placed must not be taken for none."""
+    m = block.get_submodule(path)
+    p = m._parameters.pop(name)
+    object.__setattr__(m, name, p.detach() + 1)
+    assert not block._plain_decode(64)
+    m._parameters[name] = p
+    assert not block._plain_decode(64)
+    object.__delattr__(m, name)
+    assert block._plain_decode(64)
+    m._parameters.pop(name)
+    m.register_buffer(name, p.detach() + 1)
+    assert not block._plain_decode(64)
+
+
+def test_a_linear_without_bias_stays_plain(block):
+    block.attn.project = nn.Linear(64, 64, bias=False)
+    assert block._plain_decode(64)
+    block.attn.project.bias = nn.Parameter(torch.zeros(64))
+    assert block._plain_decode(64)
