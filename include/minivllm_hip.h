@@ -269,13 +269,16 @@ int64_t mgi_paged_decode_workgroup_waves(int64_t B, int64_t H, int64_t D,
  * element stride bt_stride.
  * A chunk of too few query tiles to fill the GPU (head_dim a multiple of 8;
  * in the 2-byte types only after a prefix at least as long) has its keys,
- * when a cost model says it pays, split over several workgroups per query tile and the
- * partials merged in a second pass; workspace must then hold
- * mgi_paged_prefill_workspace_bytes(...) bytes for the same (start_pos, T,
- * H, D, dtype), and it may be NULL when that is 0. A workspace that is missing
- * or smaller gets the plain split of the total key tiles over two workgroups
- * per CU (2-byte types; MGI_EWORKSPACE when that one does not fit either), or
- * no split. Its contents need no initialisation; calls that overlap in time need separate workspaces.
+ * when a cost model says it pays, split over several workgroups per query
+ * tile and the partials merged in a second pass. Workspace for it:
+ * mgi_paged_prefill_workspace_bytes(...) for the same (start_pos, T, H, D,
+ * dtype), 16-byte aligned; NULL will do when that is 0. A call whose
+ * workspace is missing, smaller or misaligned takes, in the 2-byte types, the
+ * plain split (the total key tiles over two workgroups per CU), which block
+ * sizes below 16 or not a power of two always take, or fails (MGI_EWORKSPACE;
+ * MGI_EINVAL when misaligned) if that one has no room either; where there is
+ * no plain split, and in fp32, it runs unsplit. Contents need no
+ * initialisation; calls that overlap in time need separate workspaces.
  * MINIVLLM_HIP_PREFILL_SPLIT_KEYS (read on every call, by both functions)
  * turns the split off (-1) or forces that many keys per partition (> 0; fp32
  * then runs unsplit).

@@ -351,11 +351,11 @@ struct PrefillSplit {
 // spread over the XCDs. `plain`, the split with one partition length (total
 // tiles over two per CU), stays unless a candidate is 7 % cheaper: nearer
 // than that the estimates don't tell them apart. Measured on MI355X, plain
-// / this (us, bf16, D = 128): 300 rows after 15 000, 32 heads: 183 / 117;
-// 640 after 15 000: 226 / 186; 400 after 6000, 20 heads: 86 / 55; 900 after
-// 3000, 16 heads: 59 / 46; 450 after 5000, 32 heads: 66 / 58; 1100 after
-// 5000, 12 heads: 83 / 66; 500 after 10 000, 12 heads, D = 64: 47 / 37;
-// 1500 after 11 700, 12 heads: 190 / 158.
+// / this (us, bf16, D = 128, replayed from a graph): 300 rows after 15 000, 32
+// heads: 177 / 136; 640 after 15 000: 214 / 195; 400 after 6000, 20 heads:
+// 87 / 59; 900 after 3000, 16 heads: 59 / 55; 450 after 5000, 32 heads: 66 /
+// 63; 1100 after 5000, 12 heads: 80 / 66; 500 after 10 000, 12 heads, D = 64:
+// 47 / 37; 1500 after 11 700, 12 heads: 190 / 146.
 PrefillSplit cheapest_prefill_split(int64_t start, int64_t T, int64_t H, int64_t D, const PrefillSplit& plain) {
   struct Config {
     int cfg, rows, per_cu;
@@ -540,7 +540,9 @@ int64_t mgi_paged_decode_workgroup_waves(int64_t B, int64_t H, int64_t D, int64_
 
 size_t mgi_paged_prefill_workspace_bytes(int64_t start_pos, int64_t T, int64_t H, int64_t D, int dtype) {
   if (start_pos < 0 || T <= 0 || H <= 0 || D <= 0 || !valid_dtype(dtype)) return 0;
-  return prefill_workspace(start_pos, T, H, D, dtype, false).total;
+  const size_t priced = prefill_workspace(start_pos, T, H, D, dtype, false).total;
+  // Strides and block size are not known here: room for the plain split too.
+  return dtype == MGI_F32 ? priced : std::max(priced, prefill_workspace(start_pos, T, H, D, dtype, true).total);
 }
 
 size_t mgi_paged_decode_workspace_bytes(int64_t B, int64_t H, int64_t D, int64_t S, int64_t M,
@@ -1080,9 +1082,15 @@ int mgi_paged_prefill(void* out, const int64_t* out_strides, const void* q,
     // bf16 chunk of 16 heads, as each thread then stages twice the tile.)
     a.cus = device_cus();
     const int waves = T <= 32 ? 2 : 4;
-    // A caller without room for the priced split (one that sizes its workspace
-    // for the plain one, or gives none) gets the plain split, or none.
-    PrefillWorkspace pw = prefill_workspace(start_pos, T, H, D, dtype, false);
+    // The prices describe the direct-to-LDS kernel: other calls (block sizes
+    // below 16 or not a power of two, large strides) keep the plain split, as on
+    // their 64-row tiles the priced lengths run 5-11 % slower where they are
+    // meant for 128 rows (us, S = 8, plain / priced: 450 rows after 5000, 32
+    // heads, 94.7 / 99.1; 500 after 10 000, 12 heads, D = 64, 59.4 / 65.9). A
+    // caller without room for the priced split (one that sizes its workspace for
+    // the plain one, or gives none) gets the plain split, or none.
+    PrefillWorkspace pw =
+        prefill_workspace(start_pos, T, H, D, dtype, dtype != MGI_F32 && !prefill_direct_to_lds(a, dp));
     if (pw.part_keys > 0 && (!workspace || workspace_bytes < pw.total || !aligned16(workspace)))
       pw = prefill_workspace(start_pos, T, H, D, dtype, true);
     if (pw.part_keys > 0) {

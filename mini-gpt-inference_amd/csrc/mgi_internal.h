@@ -158,6 +158,9 @@ hipError_t launch_paged_decode(const DecodeArgs& a, int dtype, const DecodePlan&
 int prefill_head_dim_bucket(int two_byte, int D);
 hipError_t launch_paged_prefill(const PrefillArgs& a, int dtype, int dp, int waves, int qpw,
                                 hipStream_t stream);
+// Whether that launch of a 2-byte type takes the direct-to-LDS kernel
+// (paged_prefill_tr), whose workgroups the key split's prices describe.
+bool prefill_direct_to_lds(const PrefillArgs& a, int dp);
 
 // paged_decode_merge alone (partition mode), for partials another kernel wrote
 // in its layout; `lanes_per_head` as in DecodePlan.

@@ -1422,6 +1422,10 @@ hipError_t launch_dp(const PrefillArgs& a, int waves, int qpw, hipStream_t strea
 
 }  // namespace
 
+bool prefill_direct_to_lds(const PrefillArgs& a, int dp) {
+  return (dp == 64 || dp == 128) && a.T > 32 && prefill_tr_mode() != 0 && tr_eligible(a);
+}
+
 int prefill_head_dim_bucket(int two_byte, int D) {
   if (D <= 32) return 32;
   if (D <= 64) return 64;

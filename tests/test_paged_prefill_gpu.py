@@ -527,3 +527,31 @@ def test_priced_key_split_agrees_with_unsplit(monkeypatch, start, T, H, D, dtype
     err = ((out - whole).norm() / whole.norm()).item()
     print(f"  split against unsplit: {err:.2e}", flush=True)
     assert err <= (2.0 ** -8 if dtype == torch.bfloat16 else 2.0 ** -11)
+
+
+def plain_split_keys(start, T, H):
+    """Keys per partition of the plain split: a chunk's key tiles, over its 64-row
+    query tiles, shared out over two workgroups per CU."""
+    total = sum(-(-(start + min(T, r + 64)) // 64) for r in range(0, T, 64))
+    slots = 2 * torch.cuda.get_device_properties(0).multi_processor_count
+    return 64 * max(2, -(-total * H // slots))
+
+
+@pytest.mark.parametrize("S", [4, 8, 24, 16])
+@pytest.mark.parametrize("start,T,H,D", [(5000, 450, 32, 128), (10000, 500, 12, 64), (15000, 300, 32, 128)])
+def test_block_sizes_the_prices_do_not_describe_take_the_plain_split(start, T, H, D, S, monkeypatch):
+    """Key split prices hold for the direct-to-LDS kernel; calls on other block
+    sizes have the bits of the plain partition length, as calls on its own (16)
+    do not."""
+    dtype = torch.bfloat16
+    n = -(-(start + T) // S)
+    g = torch.Generator(device=DEV).manual_seed(T)
+    pool = KVBlockPool(1, n, S, H, D, device=DEV, dtype=dtype)
+    pool.k.normal_(generator=g)
+    pool.v.normal_(generator=g)
+    table = torch.randperm(n, generator=torch.Generator().manual_seed(T))
+    q = torch.randn((T, H, D), generator=g, device=DEV).to(dtype)
+    out = run_hip(q, pool, table, start, 0)
+    monkeypatch.setenv("MINIVLLM_HIP_PREFILL_SPLIT_KEYS", str(plain_split_keys(start, T, H)))
+    plain = run_hip(q, pool, table, start, 0)
+    assert torch.equal(out, plain) == (S != 16)
