@@ -280,11 +280,40 @@ int next_pow2_at_least4(int64_t x) {
 // partitions of pk keys, counted once per partition they span.
 int64_t split_partials(int64_t start, int64_t T, int64_t pk) {
   int64_t n = 0;
-  for (int64_t j = 2; (j - 1) * pk < start + T; ++j) {
+  for (int64_t j = std::max<int64_t>(2, start / pk + 1); (j - 1) * pk < start + T; ++j) {
     const int64_t lo = std::max(start + 1, (j - 1) * pk + 1), hi = std::min(start + T, j * pk);
     if (hi >= lo) n += (hi - lo + 1) * j;
   }
   return n;
+}
+
+// Sum of floor(j / k) over 0 <= j < x.
+int64_t floor_sum(int64_t x, int64_t k) {
+  const int64_t q = x / k, r = x % k;
+  return k * (q * (q - 1) / 2) + q * r;
+}
+
+// Workgroups per head of a chunk whose query tiles of `rows` rows (64, 128, or
+// all of a shorter chunk) have their 64-key tiles cut into partitions of k: the
+// sum of ceil(tiles / k). A closed form, as the prices below ask it for many k on
+// every call (summed tile by tile, 4000 rows after 16 384, 4 heads, D = 64, took
+// 53 us of host time a query; so, 10): with s tiles of prefix, tile i has m (i + 1) + s (m = rows / 64),
+// and the last one what the chunk ends with.
+int64_t key_partitions(int64_t start, int64_t T, int64_t rows, int64_t k) {
+  const int64_t m = std::max<int64_t>(1, rows / 64), n = (T + rows - 1) / rows - 1;  // all but the last
+  const int64_t last = ((start + T + 63) / 64 + k - 1) / k;
+  const int64_t c = m + (start + 63) / 64 + k - 1;  // sum of floor((m i + c) / k) over 0 <= i < n
+  if (n == 0) return last;
+  const int64_t each = floor_sum(c + m * n, k) - floor_sum(c, k);  // ... of floor(j / k) over c <= j < c + m n
+  if (m == 1) return each + last;
+  // Every second j: a pair (j, j + 1) differs, by one, where k divides j + 1 = 2 i + c + 1.
+  int64_t pairs = 0;
+  if (k % 2 == 1 || c % 2 == 1) {
+    const int64_t period = k % 2 ? k : k / 2;
+    const int64_t i0 = k % 2 ? (k - (c + 1) % k) * ((k + 1) / 2) % k : (period - (c + 1) / 2 % period) % period;
+    pairs = i0 < n ? (n - 1 - i0) / period + 1 : 0;
+  }
+  return (each - pairs) / 2 + last;
 }
 
 // Paged prefill key split of the fp32 kernel. Its workgroups run one 64-key
@@ -307,18 +336,14 @@ int64_t prefill_split_keys_f32(int64_t start, int64_t T, int64_t H, int64_t D) {
   const int dp = mgi::prefill_head_dim_bucket(0, (int)D);
   if (D % 8 != 0 || dp == 0 || T <= 0 || start + T > kMaxSplitKeysF32) return 0;
   const int64_t QB = T <= 32 ? 32 : 64, nq = (T + QB - 1) / QB;
-  auto tiles = [&](int64_t qt) { return (start + std::min(T, (qt + 1) * QB) + 63) / 64; };
   if (nq * H >= 8 * (int64_t)device_cus()) return 0;  // rounds enough to even out
   const double cus = (double)device_cus(), tile_us = dp == 32 ? 2.4 : dp == 64 ? 3.5 : 7.5;
-  int64_t total = 0;
-  for (int64_t qt = 0; qt < nq; ++qt) total += tiles(qt);
-  const double share = (double)(total * H) / cus;
+  const double share = (double)(key_partitions(start, T, QB, 1) * H) / cus;
   auto cost = [&](int64_t k) {  // k tiles per partition
-    int64_t wgs = 0;
-    for (int64_t qt = 0; qt < nq; ++qt) wgs += (tiles(qt) + k - 1) / k;
-    return tile_us * std::max((double)k, share + 0.5 * (double)k) + 2.0 * (double)(wgs * H) / cus;
+    const int64_t wgs = key_partitions(start, T, QB, k) * H;
+    return tile_us * std::max((double)k, share + 0.5 * (double)k) + 2.0 * (double)wgs / cus;
   };
-  const int64_t longest = tiles(nq - 1);
+  const int64_t longest = (start + T + 63) / 64;
   double best_us = 0.9 * cost(longest);  // nearer than that, either may win
   int64_t best = 0;
   for (int64_t k = 1; k < longest; k += std::max<int64_t>(1, k / 8)) {
@@ -369,9 +394,7 @@ PrefillSplit cheapest_prefill_split(int64_t start, int64_t T, int64_t H, int64_t
   };
   const int64_t cus = device_cus(), n = (start + T + 63) / 64, w64 = (T + 63) / 64 * H;
   auto wgs_of = [&](const Config& c, int64_t k) {  // workgroups with partitions of k tiles
-    int64_t w = 0;
-    for (int64_t q0 = 0; q0 < T; q0 += c.rows) w += ((start + std::min(T, q0 + c.rows) + 63) / 64 + k - 1) / k;
-    return w * H;
+    return key_partitions(start, T, c.rows, k) * H;
   };
   auto cost = [&](const Config& c, int64_t k) {
     const int64_t wgs = wgs_of(c, k);
@@ -390,7 +413,11 @@ PrefillSplit cheapest_prefill_split(int64_t start, int64_t T, int64_t H, int64_t
       if (fill * cus < 2 * ((T + c.rows - 1) / c.rows) * H) continue;
       // The shortest partitions whose workgroups fit: from the mean up.
       int64_t k = std::max<int64_t>(2, wgs_of(c, 1) / (fill * cus));
-      while (k < n && wgs_of(c, k) > fill * cus) ++k;
+      for (int64_t hi = n; k < hi;) {  // the first k whose workgroups fit, or n
+        const int64_t mid = k + (hi - k) / 2;
+        if (wgs_of(c, mid) > fill * cus) k = mid + 1;
+        else hi = mid;
+      }
       if (k >= n || (n + k - 1) / k > kMaxGridYZ) continue;
       const double us = cost(c, k);
       if (us < best_us) {
@@ -423,12 +450,7 @@ PrefillSplit prefill_split(int64_t start, int64_t T, int64_t H, int64_t D, int d
   if (forced < 0 || D % 8 != 0 || dp == 0 || T <= 0 || T > kMaxGridYZ) return {};
   const int64_t QB = T <= 32 ? 32 : 64;
   const int64_t nq = (T + QB - 1) / QB;
-  int64_t total = 0, longest = 0;
-  for (int64_t qt = 0; qt < nq; ++qt) {
-    const int64_t tiles = (start + std::min(T, (qt + 1) * QB) + 63) / 64;
-    total += tiles;
-    longest = std::max(longest, tiles);
-  }
+  const int64_t total = key_partitions(start, T, QB, 1), longest = (start + T + 63) / 64;
   if (forced > 0) {
     const int64_t pk = round_up(forced, 64);
     return {pk < longest * 64 && (start + T + pk - 1) / pk <= kMaxGridYZ ? pk : 0, 0};  // partitions: grid y

@@ -5,6 +5,7 @@ from __future__ import annotations
 
 import ctypes
 import re
+import time
 from pathlib import Path
 
 import pytest
@@ -117,6 +118,47 @@ def test_split_tokens_and_workspace_sizes():
 def _prefill_ws(monkeypatch, split_keys, start, T, H, D, dtype=1):
     monkeypatch.setenv("MINIVLLM_HIP_PREFILL_SPLIT_KEYS", str(split_keys))
     return _native.lib().mgi_paged_prefill_workspace_bytes(start, T, H, D, dtype)
+
+
+def test_plain_prefill_split_matches_a_count_tile_by_tile(monkeypatch):
+    """Head dims without a priced split: the plain split's partition length from
+    the key tiles of each 64-row query tile, counted one by one (256 CUs when no
+    device is visible, as on MI355X)."""
+    monkeypatch.delenv("MINIVLLM_HIP_PREFILL_SPLIT_KEYS", raising=False)
+    f, D, split = _native.lib().mgi_paged_prefill_workspace_bytes, 32, 0
+    for start, T, H in [(s, t, h) for s in (63, 64, 65, 1000, 4095, 16384, 100001) for t in (1, 32, 33, 64, 65, 200, 999)
+                        for h in (1, 3, 8, 20) if s >= t]:
+        rows = 32 if T <= 32 else 64
+        tiles = [-(-(start + min(T, r + rows)) // 64) for r in range(0, T, rows)]
+        k = max(2, -(-sum(tiles) * H // 512))
+        want = 0
+        if len(tiles) * H < 512 and k < tiles[-1]:
+            spans = sum(p for p in (-(-(start + i + 1) // (64 * k)) for i in range(T)) if p > 1)
+            if k * 0.75 + 8.0 + 2.0 * spans * H * (4 * D + 8) / 5.0e6 < tiles[-1] * 0.75:
+                n = T * H * -(-(start + T) // (64 * k))
+                want = -(-n * D * 4 // 256) * 256 + n * 8
+        assert f(start, T, H, D, _native.MGI_BF16) == want, (start, T, H)
+        split += want > 0
+    assert split > 50
+
+
+def test_prefill_split_prices_do_not_grow_with_the_chunk(monkeypatch):
+    """Every prefill call prices its split (twice, with the workspace query):
+    the host time of that does not grow with the chunk's query tiles."""
+    monkeypatch.delenv("MINIVLLM_HIP_PREFILL_SPLIT_KEYS", raising=False)
+
+    def least(*args):
+        best = float("inf")
+        for _ in range(30):
+            t0 = time.perf_counter()
+            for _ in range(50):
+                _native.lib().mgi_paged_prefill_workspace_bytes(*args)
+            best = min(best, time.perf_counter() - t0)
+        return best
+
+    # 14 and 4.4 times when summed tile by tile
+    assert least(16384, 8000, 2, 64, _native.MGI_BF16) < 3 * least(16384, 400, 2, 64, _native.MGI_BF16)
+    assert least(10000, 5000, 4, 64, _native.MGI_F32) < 2.5 * least(10000, 500, 4, 64, _native.MGI_F32)
 
 
 def test_prefill_split_workspace_sizes(monkeypatch):
