@@ -61,8 +61,9 @@ const char* mgi_last_error(void);
  * mgi_paged_decode_balanced_waves and the even split of split_tokens = 0;
  * 1.02 the prefill key split (mgi_paged_prefill's workspace arguments and
  * mgi_paged_prefill_workspace_bytes); 1.03 mgi_paged_decode_noalloc; 1.04
- * mgi_paged_decode_append. mgi_decode_linear, mgi_decode_linear_norm and
- * mgi_paged_decode_workgroup_waves came later without a change to the others. */
+ * mgi_paged_decode_append. mgi_decode_linear, mgi_decode_linear_norm, their
+ * queries and mgi_paged_decode_workgroup_waves came later without a change to
+ * the others. */
 int mgi_abi_version(void);
 
 /*
@@ -314,6 +315,10 @@ size_t mgi_paged_prefill_workspace_bytes(int64_t start_pos, int64_t T,
  */
 int mgi_decode_linear(void* out, const void* x, const void* weight, const void* bias,
                       int gelu, int dtype, int64_t B, int64_t N, int64_t K, void* stream);
+
+/* Whether mgi_decode_linear takes these sizes and callers with another linear
+ * layer (and GELU) at hand should call it, as measured against PyTorch's. */
+int mgi_decode_linear_pays(int64_t B, int64_t N, int64_t K, int gelu);
 
 /*
  * The projection back to the residual stream and the LayerNorm that follows:

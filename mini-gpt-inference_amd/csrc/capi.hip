@@ -979,6 +979,22 @@ int mgi_decode_linear(void* out, const void* x, const void* weight, const void* 
   return MGI_OK;
 }
 
+// More than 48 rows of more than 1536 go to PyTorch's linear. Measured on MI355X
+// (us, this / PyTorch; bf16, weights from memory, replayed from a graph): 64 rows,
+// K = 2048, to 6144: 15.6 / 13.1 (48: 13.6 / 13.2; 40: 13.0 / 13.3); K = 2560, to
+// 7680: 18.9 / 16.3 (48: 16.6 / 16.2). With GELU they stay (64 rows, K = 2048, to
+// 8192: 17.6 / 16.8, but one launch for two: the block's step 86 / 98), as does K =
+// 1536 (64 rows, to 4608: 11.9 / 10.6, the block's step 71 / 82: the host's cost of
+// the PyTorch calls) and a wide vocabulary on a narrow model (16 rows, K = 512, to
+// 50 257: 26.4 / 15.3, K = 1024: 33.9 / 22.4, but a step of 2 layers 117 / 145 and
+// 131 / 148 us when not replayed from a graph).
+int mgi_decode_linear_pays(int64_t B, int64_t N, int64_t K, int gelu) {
+  using namespace mgi;
+  if (B < 1 || B > kLinearMaxRows || N < 1 || N >= (int64_t(1) << 30) || K < 64 || K > kLinearMaxK || K % 64 != 0)
+    return 0;
+  return gelu || B <= 48 || K <= 1536;
+}
+
 size_t mgi_decode_linear_norm_workspace_bytes(int64_t B, int64_t N, int64_t K) {
   if (B <= 0 || N <= 0 || K <= 0) return 0;
   return (size_t)(linear_splits(K, nullptr) * B * N * 4);

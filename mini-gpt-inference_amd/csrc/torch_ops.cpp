@@ -220,16 +220,15 @@ void* ptr(const c10::optional<at::Tensor>& t) { return t ? t->data_ptr() : nullp
 
 constexpr int64_t kLinearRows = 64;
 
-// decode_linear(x, weight, bias, gelu): act(x W^T + bias) for x [B, 1, K] -> [B, 1, N]; None when the call is not one the kernel takes
-// (the caller then makes the PyTorch calls it stands for).
+// decode_linear(x, weight, bias, gelu): act(x W^T + bias) for x [B, 1, K] -> [B,
+// 1, N]; None when the kernel does not take the call, or PyTorch's calls are the
+// faster ones (the caller then makes those).
 py::object decode_linear(const at::Tensor& x, const at::Tensor& w, const c10::optional<at::Tensor>& bias,
                          bool gelu) {
   if (!x.is_cuda() || x.dim() != 3 || x.size(1) != 1 || w.dim() != 2) return py::none();
   const int64_t B = x.size(0), K = x.size(2), N = w.size(0);
   const int dt = dtype_code(x.scalar_type());
-  if ((dt != MGI_BF16 && dt != MGI_F16) || B < 1 || B > kLinearRows || K < 64 || K % 64 != 0 || K > 2560 || N < 1 ||
-      w.size(1) != K || (B > 48 && K > 1536 && !gelu))
-    return py::none();
+  if ((dt != MGI_BF16 && dt != MGI_F16) || w.size(1) != K || !mgi_decode_linear_pays(B, N, K, gelu)) return py::none();
   if (!linear_ok(x, x, B * K) || !linear_ok(w, x, N * K) || !linear_ok(bias, x, N))
     return py::none();
   at::Tensor out = at::empty({B, 1, N}, x.options());

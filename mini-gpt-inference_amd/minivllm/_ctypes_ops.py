@@ -1,4 +1,4 @@
-"""The eager path's four calls through ctypes, for when the _hip_ops
+"""The eager path's calls through ctypes, for when the _hip_ops
 extension (csrc/torch_ops.cpp) cannot be loaded but libminivllm_hip.so can,
 for example after a PyTorch update that the extension was not rebuilt for.
 
@@ -205,3 +205,69 @@ def paged_prefill(q: torch.Tensor, kp: torch.Tensor, vp: torch.Tensor, bt: torch
         h, d, S, N, L, int(layer_idx), 1.0 / math.sqrt(d),
         ws.data_ptr() if ws is not None else None, ws_bytes, _native.stream_handle(q.device)))
     return out
+
+
+def _linear_ok(t: torch.Tensor | None, x: torch.Tensor, numel: int) -> bool:
+    """Whether t (or no tensor) is plain, contiguous and 16-byte aligned, of x's
+    dtype and (current) device, with numel elements."""
+    return t is None or (t.dtype == x.dtype and t.device == x.device and t.numel() == numel
+                         and t.device.index == torch.cuda.current_device() and t.layout == torch.strided
+                         and t.is_contiguous() and not t.is_neg() and t.data_ptr() % 16 == 0)
+
+
+def _ptr(t: torch.Tensor | None):
+    return None if t is None else t.data_ptr()
+
+
+def decode_linear(x: torch.Tensor, w: torch.Tensor, bias: torch.Tensor | None, gelu: bool) -> torch.Tensor | None:
+    """act(x W^T + bias), [B, 1, K] -> [B, 1, N], or None when the call is not
+    one to make."""
+    if not x.is_cuda or x.ndim != 3 or x.shape[1] != 1 or w.ndim != 2 \
+            or x.dtype not in (torch.bfloat16, torch.float16):
+        return None
+    b, k, n = x.shape[0], x.shape[2], w.shape[0]
+    lib = _native.lib()
+    if w.shape[1] != k or not lib.mgi_decode_linear_pays(b, n, k, int(gelu)) or not _linear_ok(x, x, b * k) \
+            or not _linear_ok(w, x, n * k) or not _linear_ok(bias, x, n):
+        return None
+    out = torch.empty((b, 1, n), dtype=x.dtype, device=x.device)
+    _native.check(lib.mgi_decode_linear(out.data_ptr(), x.data_ptr(), w.data_ptr(), _ptr(bias), int(gelu),
+                                        _native.DTYPE_CODES[x.dtype], b, n, k, _native.stream_handle(x.device)))
+    return out
+
+
+def decode_linear_norm(x: torch.Tensor | None, w: torch.Tensor | None, bias: torch.Tensor | None,
+                       residual: torch.Tensor, ln_w: torch.Tensor | None, ln_b: torch.Tensor | None, ln_eps: float):
+    """(h, LN(h)) with h = x W^T + bias + residual, or (h, None) without the
+    LayerNorm pair; without x and w (residual, LN(residual)). None when the call
+    is not one the kernel takes."""
+    r = residual
+    if not r.is_cuda or r.ndim != 3 or r.shape[1] != 1 or r.dtype not in (torch.bfloat16, torch.float16) \
+            or (x is None) != (w is None) or (ln_w is None) != (ln_b is None) or (x is None and ln_w is None):
+        return None
+    b, n = r.shape[0], r.shape[2]
+    if not 1 <= b <= 64 or not 4 <= n <= 4096 or n % 4 != 0:
+        return None
+    k = 0
+    if x is not None:
+        if x.ndim != 3 or x.shape[0] != b or x.shape[1] != 1 or w.ndim != 2:
+            return None
+        k = x.shape[2]
+        if k < 64 or k % 64 != 0 or tuple(w.shape) != (n, k) or not _linear_ok(x, r, b * k) \
+                or not _linear_ok(w, r, n * k):
+            return None
+    if not _linear_ok(r, r, b * n) or not all(_linear_ok(t, r, n) for t in (bias, ln_w, ln_b)):
+        return None
+    lib = _native.lib()
+    out = norm = ws = None
+    ws_bytes = 0
+    if x is not None:
+        out = torch.empty((b, 1, n), dtype=r.dtype, device=r.device)
+        ws_bytes = int(lib.mgi_decode_linear_norm_workspace_bytes(b, n, k))
+        ws = torch.empty(ws_bytes, dtype=torch.uint8, device=r.device)
+    if ln_w is not None:
+        norm = torch.empty((b, 1, n), dtype=r.dtype, device=r.device)
+    _native.check(lib.mgi_decode_linear_norm(
+        _ptr(out), _ptr(norm), _ptr(x), _ptr(w), _ptr(bias), r.data_ptr(), _ptr(ln_w), _ptr(ln_b), float(ln_eps),
+        _native.DTYPE_CODES[r.dtype], b, n, k, _ptr(ws), ws_bytes, _native.stream_handle(r.device)))
+    return (r if out is None else out), norm

@@ -41,6 +41,7 @@ EXPORTED_SYMBOLS = (
     "mgi_paged_prefill",
     "mgi_paged_prefill_workspace_bytes",
     "mgi_decode_linear",
+    "mgi_decode_linear_pays",
     "mgi_decode_linear_norm",
     "mgi_decode_linear_norm_workspace_bytes",
 )
@@ -123,6 +124,8 @@ def _declare(lib: ctypes.CDLL) -> None:
         _p, _p, _p, _p, _i, _i,            # out, x, weight, bias, gelu, dtype
         _i64, _i64, _i64, _p,              # B N K, stream
     ]
+    lib.mgi_decode_linear_pays.restype = _i
+    lib.mgi_decode_linear_pays.argtypes = [_i64, _i64, _i64, _i]
     lib.mgi_decode_linear_norm.restype = _i
     lib.mgi_decode_linear_norm.argtypes = [
         _p, _p, _p, _p, _p, _p,            # out, norm, x, weight, bias, residual
@@ -156,9 +159,9 @@ def lib() -> ctypes.CDLL:
 
 
 def ops():
-    """The eager path's binding: kv_append, paged_decode, paged_decode_append
-    and paged_prefill on tensors, validated, calling the C ABI on the current
-    stream.
+    """The eager path's binding: kv_append, paged_decode, paged_decode_append,
+    paged_prefill, decode_linear and decode_linear_norm on tensors, validated,
+    calling the C ABI on the current stream.
 
     Normally the PyTorch extension _hip_ops (csrc/torch_ops.cpp). When the
     library loads but the extension does not (missing, or built against

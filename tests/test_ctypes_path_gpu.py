@@ -66,6 +66,36 @@ def test_ctypes_path_is_bit_identical_to_the_extension(dtype):
         assert torch.equal(_bits(a), _bits(b))
 
 
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16], ids=["bf16", "f16"])
+def test_decode_linear_calls_are_bit_identical_and_take_the_same(dtype):
+    """The decode step's linear calls: the same bits, and None for the same calls."""
+    ext = _native._load_extension()
+    print(f"  ctypes decode_linear against _hip_ops, {dtype}", flush=True)
+    g = torch.Generator(device=DEV).manual_seed(1)
+    make = lambda *s: torch.randn(s, generator=g, device=DEV).to(dtype)
+    x, w, bias, r, lw, lb = make(5, 1, 128), make(64, 128), make(64), make(5, 1, 64), make(64), make(64)
+    odd = make(5 * 128 + 4)[4:].view(5, 1, 128)          # 8 bytes off a 16-byte line
+    linear = [(x, w, bias, True), (x, w, None, False), (odd, w, None, False), (x.float(), w.float(), None, False),
+              (x, w, bias[:63], False), (x[:, 0], w, None, False), (x, w.t().contiguous().t(), None, False),
+              (x.cpu(), w, None, False), (make(65, 1, 128), w, None, False), (make(64, 1, 1600), make(64, 1600), None, False)]
+    norm = [(x, w, bias, r, lw, lb, 1e-5), (x, w, None, r, None, None, 0.0), (None, None, None, r, lw, lb, 1e-5),
+            (x, None, None, r, lw, lb, 1e-5), (x, w, None, r, lw, None, 1e-5), (None, None, None, r, None, None, 0.0),
+            (x, w, None, r[:4], None, None, 0.0), (odd, w, None, r, None, None, 0.0), (x, w, None, r, lw.float(), lb, 0.0)]
+    taken = 0
+    with torch.inference_mode():
+        for fn, calls in (("decode_linear", linear), ("decode_linear_norm", norm)):
+            for i, args in enumerate(calls):
+                a, b = getattr(ext, fn)(*args), getattr(_ctypes_ops, fn)(*args)
+                torch.cuda.synchronize()
+                assert (a is None) == (b is None), (fn, i)
+                if a is None:
+                    continue
+                taken += 1
+                for p, q in zip(a, b) if isinstance(a, tuple) else [(a, b)]:
+                    assert (p is None) == (q is None) and (p is None or torch.equal(_bits(p), _bits(q))), (fn, i)
+    assert taken == 2 + 3
+
+
 def test_ctypes_path_raises_the_extension_messages():
     ext = _native._load_extension()
     pool, tables, ctx, qkv = _case(torch.bfloat16)

@@ -51,6 +51,7 @@ def test_decode_linear(K, N, dtype):
             if B > 48 and K > 1536 and not gelu:
                 assert y is None
                 continue
+            assert _native.lib().mgi_decode_linear_pays(B, N, K, gelu) == 1
             want = x.double() @ w.double().t().contiguous() + (0 if b is None else b.double())
             close(y, F.gelu(want) if gelu else want, 1, dtype)
 

@@ -38,8 +38,10 @@ def test_torch_binding_loads_and_validates_on_the_host():
     and raises the wrappers' ValueErrors before any device work: CPU tensors
     are refused first."""
     ops = _native.ops()
-    for name in ("kv_append", "paged_decode", "paged_decode_append", "paged_prefill"):
-        assert callable(getattr(ops, name)), name
+    from minivllm import _ctypes_ops
+    for name in ("kv_append", "paged_decode", "paged_decode_append", "paged_prefill", "decode_linear",
+                 "decode_linear_norm"):
+        assert callable(getattr(ops, name)) and callable(getattr(_ctypes_ops, name)), name
     from minivllm import hip_paged_decode as hpd
     from minivllm.kv_block_pool import KVBlockPool
 
@@ -360,3 +362,11 @@ def test_noalloc_decode_refuses_splits_beyond_its_scratch_on_host():
     assert st == _native.MGI_EUNSUPPORTED
     msg = lib.mgi_last_error().decode()
     assert "scratch" in msg and str(32 << 20) in msg
+
+
+@pytest.mark.parametrize("B,N,K,gelu,pays", [
+    (16, 50257, 512, 0, 1), (1, 1, 64, 0, 1), (64, 50257, 1024, 0, 1), (64, 6144, 1600, 0, 0), (64, 10240, 2560, 1, 1),
+    (48, 6144, 2048, 0, 1), (49, 6144, 2048, 0, 0), (64, 8192, 2048, 1, 1), (64, 4608, 1536, 0, 1),
+    (65, 512, 512, 0, 0), (0, 512, 512, 0, 0), (8, 512, 2624, 0, 0), (8, 512, 100, 0, 0), (8, 0, 512, 0, 0), (8, 1 << 30, 512, 0, 0)])
+def test_decode_linear_sizes_that_pay(B, N, K, gelu, pays):
+    assert _native.lib().mgi_decode_linear_pays(B, N, K, gelu) == pays
