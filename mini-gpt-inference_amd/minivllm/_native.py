@@ -153,7 +153,11 @@ def lib() -> ctypes.CDLL:
                 handle = ctypes.CDLL(str(path))
             except OSError as exc:
                 raise RuntimeError(f"HIP extension failed to load: {exc}") from exc
-            _declare(handle)
+            try:
+                _declare(handle)
+            except AttributeError as exc:
+                raise RuntimeError(f"HIP extension is out of date: {path}: {exc} "
+                                   "(run `python -c 'import __graft_entry__ as g; g.build()'` at the repo root)") from exc
             _lib = handle
     return _lib
 

@@ -5,6 +5,7 @@ from __future__ import annotations
 
 import ctypes
 import re
+import subprocess
 import time
 from pathlib import Path
 
@@ -95,6 +96,21 @@ def test_missing_library_is_an_error_not_a_fallback(monkeypatch, tmp_path):
     monkeypatch.setattr(_native, "library_path", lambda: tmp_path / "libminivllm_hip_missing.so")
     with pytest.raises(RuntimeError, match="HIP extension not built"):
         _native.ops()
+
+
+def test_library_without_a_declared_symbol_is_out_of_date(monkeypatch, tmp_path):
+    """A library built before the header's newest entry points: RuntimeError
+    naming it, as for a missing one, and nothing is kept."""
+    src = tmp_path / "old.c"
+    src.write_text("".join(f"void {n}(void) {{}}\n" for n in _native.EXPORTED_SYMBOLS if "decode_linear" not in n))
+    old = tmp_path / "libminivllm_hip_old.so"
+    subprocess.run(["gcc", "-shared", "-fPIC", "-o", str(old), str(src)], check=True)
+    monkeypatch.setattr(_native, "_ops", None)
+    monkeypatch.setattr(_native, "_lib", None)
+    monkeypatch.setattr(_native, "library_path", lambda: old)
+    with pytest.raises(RuntimeError, match="out of date.*mgi_decode_linear"):
+        _native.ops()
+    assert _native._lib is None
 
 
 def test_split_tokens_and_workspace_sizes():
