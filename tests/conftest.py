@@ -28,3 +28,10 @@ def progress(request):
             print(line, flush=True)
 
     return emit
+
+
+@pytest.fixture
+def split_kernels(monkeypatch):
+    """Decode calls take the split kernels (partitions, even split), whatever
+    their size; without it small ones go to the one-launch kernel."""
+    monkeypatch.setenv("MINIVLLM_HIP_DECODE_WG", "0")

@@ -8,8 +8,9 @@ pools must be identical (the fused kernel writes a row's slot before its
 wavefront reads the block, so attention sees the same pool). Rows cover the
 decode step's cases: the slot of the sequence's last position (the fused
 write), padding (slot -1), a slot in a block no table uses, a slot past the
-pool, and a sequence with no context whose row still lands. Both splits of
-the fast kernel (even, partitions), every dtype, the lane layouts of head
+pool, and a sequence with no context whose row still lands. The kernels the
+library picks for the sizes (test_decode_split_routes_gpu.py runs the same
+cases on the split kernels, even and partitions), every dtype, the lane layouts of head
 dims 8 to 256, and the shapes that take the separate append kernel
 (generic-path head dims, rows of another dtype, a strided head dim) are
 checked; then the high-batch step at full size (B=256, 32 heads, bf16,

@@ -45,6 +45,13 @@ def hip(q, pool, tables, lens, layer, **kw):
     return out.float().cpu().numpy()
 
 
+def takes_balanced_split(B, H, D, S, M, dtype, split_tokens=0) -> bool:
+    """Whether a call of these sizes runs on the balanced split."""
+    lib, sizes = hpd._native.lib(), (B, H, D, S, M)
+    return lib.mgi_paged_decode_workgroup_waves(*sizes, hpd._native.DTYPE_CODES[dtype], split_tokens) == 0 \
+        and lib.mgi_paged_decode_balanced_waves(*sizes, split_tokens) > 0
+
+
 def oracle_args(q, pool, tables, lens, layer):
     return (fx.to_numpy(q), fx.to_numpy(pool.k), fx.to_numpy(pool.v), tables.cpu().numpy(),
             lens.cpu().numpy(), layer)
@@ -226,6 +233,7 @@ def test_decode_microbench_shape_matches_oracle(dtype):
     """B=64, H=32, D=128, S=16, ctx ~ U[512, 4096], 20k-block permuted pool."""
     print(f"  workload B=64 H=32 D=128 ctx U[512,4096] N=20000 {dtype}", flush=True)
     w = fx.make_decode_workload(64, 32, 128, 16, 20000, 512, 4096, dtype, DEV, seed=0)
+    assert takes_balanced_split(64, 32, 128, 16, w.tables.shape[1], dtype)
     _check_against_c_oracle(w, dtype)
 
 
@@ -264,7 +272,7 @@ def _set_tiers(monkeypatch, tiers):
 
 @pytest.mark.parametrize("tiers", TIERS)
 @pytest.mark.parametrize("B", [7, 200, 1000])
-def test_balanced_split_with_empty_and_one_token_contexts(B, tiers, monkeypatch):
+def test_balanced_split_with_empty_and_one_token_contexts(B, tiers, monkeypatch, split_kernels):
     """The automatic split spreads every sequence's blocks over the waves'
     own claims and the ticket claims (several sequences per claim, several
     claims per sequence); rows with no context are zeros and one-token rows
@@ -282,6 +290,7 @@ def test_balanced_split_with_empty_and_one_token_contexts(B, tiers, monkeypatch)
     assert tables.shape[1] <= M
     tables = torch.nn.functional.pad(tables, (0, M - tables.shape[1]), value=-1)
     assert hpd._native.lib().mgi_paged_decode_workspace_bytes(B, H, D, S, M, 0) > 0
+    assert takes_balanced_split(B, H, D, S, M, torch.float32)
     got = hip(q, fx.pool_to_device(pool, DEV), tables, lens, layer)
     want = c_oracle.paged_decode(*oracle_args(q, pool, tables, lens, layer))
     np.testing.assert_allclose(got, want, **F32_TOL)
@@ -289,7 +298,7 @@ def test_balanced_split_with_empty_and_one_token_contexts(B, tiers, monkeypatch)
 
 
 @pytest.mark.parametrize("B", [4096, 4100])
-def test_largest_balanced_batch_and_the_partition_fallback(B):
+def test_largest_balanced_batch_and_the_partition_fallback(B, split_kernels):
     """The balanced split holds the batch's block prefix sums in LDS, 4096
     sequences at most (64 per lane of its scan); one more row takes the
     partition split. Both against the C oracle. At this batch the library
@@ -303,7 +312,7 @@ def test_largest_balanced_batch_and_the_partition_fallback(B):
     q, pool, tables, lens, layer = _small_case(B, H, D, S, ctx.tolist(), torch.float32, seed=B, N=N)
     tables = torch.nn.functional.pad(tables, (0, M - tables.shape[1]), value=-1)
     waves = hpd._native.lib().mgi_paged_decode_balanced_waves(B, H, D, S, M, 0)
-    assert (waves > 0) == (B <= 4096), waves
+    assert (waves > 0) == (B <= 4096) == takes_balanced_split(B, H, D, S, M, torch.float32), waves
     print(f"  B={B} balanced waves per head group {waves}", flush=True)
     got = hip(q, fx.pool_to_device(pool, DEV), tables, lens, layer)
     want = c_oracle.paged_decode(*oracle_args(q, pool, tables, lens, layer))
@@ -323,7 +332,7 @@ def test_balanced_split_ignores_stale_workspace(tiers, monkeypatch):
     B, H, D = w.q.shape
     L, N, S = w.pool.k.shape[:3]
     M = w.tables.shape[1]
-    assert lib.mgi_paged_decode_balanced_waves(B, H, D, S, M, 0) > 0
+    assert takes_balanced_split(B, H, D, S, M, w.q.dtype)
     ws_bytes = int(lib.mgi_paged_decode_workspace_bytes(B, H, D, S, M, 0))
 
     def call(ws):
@@ -360,7 +369,7 @@ def test_balanced_split_ignores_stale_workspace(tiers, monkeypatch):
 
 @pytest.mark.parametrize("split", [0, 256], ids=["auto", "partitions"])
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
-def test_few_sequences_many_partials(dtype, split):
+def test_few_sequences_many_partials(dtype, split, split_kernels):
     """Few (sequence, head group) pairs with many partials each: the merge
     runs several wavefronts per workgroup (B=3, 4 heads, contexts of 5k-12k
     tokens split over hundreds of claims or 256-token partitions)."""

@@ -44,7 +44,7 @@ def _bits(t):
 
 @pytest.mark.parametrize("dtype,split", [(torch.bfloat16, 0), (torch.float32, 0), (torch.bfloat16, 256)],
                          ids=["bf16-auto", "f32-auto", "bf16-partitions"])
-def test_noalloc_matches_the_workspace_entry_on_calls_in_a_row(dtype, split):
+def test_noalloc_matches_the_workspace_entry_on_calls_in_a_row(dtype, split, split_kernels):
     lib = _native.lib()
     stream = _native.stream_handle(DEV)
     for B, lo, hi, N, seed in CALLS:
