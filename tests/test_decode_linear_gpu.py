@@ -20,8 +20,8 @@ pytestmark = pytest.mark.gpu
 DEV = torch.device("cuda:0")
 # One rounding of the stored result (half an ulp, 2^-9 and 2^-12 relative) plus f32
 # sums of K products in another order (K 2^-24 of the terms' magnitude): together
-# below one ulp of the largest output, 2^-8 and 2^-11. LayerNorm outputs add the
-# rounding of the row they normalise, so two ulps.
+# below one ulp of the largest output, 2^-8 and 2^-11. A LayerNorm is compared with
+# the float64 one of the row as it was stored, so it is one rounding too.
 ULP = {torch.bfloat16: 2.0 ** -8, torch.float16: 2.0 ** -11}
 DTYPES = [torch.bfloat16, torch.float16]
 

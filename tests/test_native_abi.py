@@ -386,3 +386,36 @@ def test_noalloc_decode_refuses_splits_beyond_its_scratch_on_host():
     (65, 512, 512, 0, 0), (0, 512, 512, 0, 0), (8, 512, 2624, 0, 0), (8, 512, 100, 0, 0), (8, 0, 512, 0, 0), (8, 1 << 30, 512, 0, 0)])
 def test_decode_linear_sizes_that_pay(B, N, K, gelu, pays):
     assert _native.lib().mgi_decode_linear_pays(B, N, K, gelu) == pays
+
+
+def test_decode_linear_entries_reject_bad_arguments():
+    """Every argument error is found on the host (made-up addresses, no device
+    work): the status, and a message for it."""
+    lib, P, BF16 = _native.lib(), 1 << 20, _native.MGI_BF16
+    INVALID, UNSUPPORTED, WORKSPACE = _native.MGI_EINVAL, _native.MGI_EUNSUPPORTED, _native.MGI_EWORKSPACE
+
+    def linear(out=P, x=P, w=P, bias=P, gelu=0, dtype=BF16, B=4, N=64, K=128):
+        return lib.mgi_decode_linear(out, x, w, bias, gelu, dtype, B, N, K, None)
+
+    def norm(out=P, norm=P, x=P, w=P, bias=P, res=P, lw=P, lb=P, dtype=BF16, B=4, N=64, K=128, ws=P, nbytes=1 << 30):
+        return lib.mgi_decode_linear_norm(out, norm, x, w, bias, res, lw, lb, 1e-5, dtype, B, N, K, ws, nbytes, None)
+
+    for call in (linear, norm):
+        for bad in (dict(B=0), dict(N=0), dict(K=0), dict(B=-1), dict(K=-64)):
+            assert call(**bad) == INVALID, bad
+        for bad in (dict(dtype=_native.MGI_F32), dict(dtype=7), dict(B=65), dict(K=100), dict(N=1 << 30), dict(K=1 << 30),
+                    dict(out=P + 8), dict(x=P + 2), dict(w=P + 8), dict(bias=P + 8)):
+            assert call(**bad) == UNSUPPORTED and lib.mgi_last_error(), bad
+    for bad in (dict(out=None), dict(x=None), dict(w=None)):
+        assert linear(**bad) == INVALID, bad
+    assert linear(K=2624) == UNSUPPORTED
+    for bad in (dict(res=None), dict(x=None), dict(w=None), dict(out=None), dict(norm=None), dict(lw=None), dict(lb=None),
+                dict(lw=None, lb=None), dict(x=None, w=None, out=None, norm=None, lw=None, lb=None), dict(x=None, w=None)):
+        assert norm(**bad) == INVALID, bad
+    for bad in (dict(N=66), dict(N=4100), dict(norm=P + 8), dict(lw=P + 8), dict(lb=P + 8), dict(res=P + 8), dict(ws=P + 8)):
+        assert norm(**bad) == UNSUPPORTED, bad
+    need = lib.mgi_decode_linear_norm_workspace_bytes(4, 64, 128)
+    assert need == 2 * 4 * 64 * 4       # two splits of one 64-wide unit, f32
+    assert norm(nbytes=need - 1) == WORKSPACE and norm(ws=None) == WORKSPACE
+    assert lib.mgi_decode_linear_norm_workspace_bytes(64, 4096, 16384) == 16 * 64 * 4096 * 4
+    assert [lib.mgi_decode_linear_norm_workspace_bytes(*s) for s in ((0, 64, 64), (4, 0, 64), (4, 64, 0))] == [0, 0, 0]

@@ -83,31 +83,87 @@ def test_rule_on_the_host(monkeypatch):
         assert len(parts) == 1
 
 
+def plain_bytes(start, T, H, D):
+    """Workspace of the 2-byte types' plain split on 256 CUs (0: none), by the
+    rule written out."""
+    tiles = [-(-(start + min(T, r + 64)) // 64) for r in range(0, T, 64)]
+    k = max(2, -(-sum(tiles) * H // 512))
+    if len(tiles) * H >= 512 or start < T or k >= tiles[-1]:
+        return 0
+    spans = sum(p for p in (-(-(start + i + 1) // (64 * k)) for i in range(T)) if p > 1)
+    tile_us = 1.5 * max(D, 64) / 128
+    if k * tile_us + 8.0 + 2.0 * spans * H * (4 * D + 8) / 5.0e6 >= tiles[-1] * tile_us:
+        return 0
+    n = T * H * -(-(start + T) // (64 * k))
+    return -(-n * D * 4 // 256) * 256 + n * 8
+
+
+def prefill_with_workspace(start, T, H, D, dtype):
+    """A bf16, f16 or fp32 call of fixed inputs as a function of its workspace
+    (bytes, and how many bytes off alignment; None for no workspace): (status,
+    output), with the bytes past the workspace checked untouched."""
+    lib, S = _native.lib(), 16
+    n = -(-(start + T) // S)
+    g = torch.Generator(device=DEV).manual_seed(T)
+    pool_k, pool_v = (torch.randn((1, n, S, H, D), generator=g, device=DEV).to(dtype) for _ in range(2))
+    q = torch.randn((T, H, D), generator=g, device=DEV).to(dtype)
+    table = torch.randperm(n, device=DEV, generator=g)
+
+    def call(nbytes, off=0):
+        print(f"  prefill start={start} T={T} H={H} D={D} {dtype} workspace {nbytes} bytes off {off}", flush=True)
+        out = torch.full_like(q, float("nan"))
+        ws = None if nbytes is None else torch.full((nbytes + 512,), 77, dtype=torch.uint8, device=DEV)
+        rc = lib.mgi_paged_prefill(
+            out.data_ptr(), _native.strides(out), q.data_ptr(), _native.strides(q), pool_k.data_ptr(), pool_v.data_ptr(),
+            _native.strides(pool_k), _native.strides(pool_v), _native.DTYPE_CODES[dtype], table.data_ptr(), 1,
+            _native.MGI_I64, n, start, T, H, D, S, n, 1, 0, D ** -0.5, None if ws is None else ws.data_ptr() + off,
+            0 if nbytes is None else nbytes, torch.cuda.current_stream().cuda_stream)
+        torch.cuda.synchronize()
+        assert ws is None or ((ws[:off] == 77).all() and (ws[off + nbytes:] == 77).all())
+        return rc, out
+    return call
+
+
 @pytest.mark.gpu
 @pytest.mark.parametrize("start,T,H", [(3000, 900, 16), (15000, 300, 32)])
-def test_bf16_workspace_too_small_for_the_priced_split(start, T, H):
-    """A workspace that holds less than the priced split's partials: the call
-    falls back to the plain split or refuses, as it did before, and never writes
-    past what it was given."""
-    lib, D, S = _native.lib(), 128, 16
-    n = -(-(start + T) // S)
-    pool_k = torch.randn((1, n, S, H, D), device=DEV).to(torch.bfloat16)
-    q = torch.randn((T, H, D), device=DEV).to(torch.bfloat16)
-    table = torch.randperm(n, device=DEV)
-    need = int(lib.mgi_paged_prefill_workspace_bytes(start, T, H, D, _native.MGI_BF16))
-    assert need > 0
-    outs = []
-    for nbytes in (need, need - 256):
-        ws = torch.full((need,), 77, dtype=torch.uint8, device=DEV)
-        out = torch.empty_like(q)
-        rc = lib.mgi_paged_prefill(
-            out.data_ptr(), _native.strides(out), q.data_ptr(), _native.strides(q), pool_k.data_ptr(), pool_k.data_ptr(),
-            _native.strides(pool_k), _native.strides(pool_k), _native.MGI_BF16, table.data_ptr(), 1, _native.MGI_I64, n,
-            start, T, H, D, S, n, 1, 0, D ** -0.5, ws.data_ptr(), nbytes, torch.cuda.current_stream().cuda_stream)
-        torch.cuda.synchronize()
-        assert rc in (_native.MGI_OK, _native.MGI_EWORKSPACE) and (nbytes < need or rc == _native.MGI_OK)
-        assert (ws[nbytes:] == 77).all()
-        if rc == _native.MGI_OK:
-            outs.append(out.double())
-    if len(outs) == 2:
-        assert ((outs[0] - outs[1]).norm() / outs[0].norm()).item() <= 2.0 ** -8
+def test_bf16_workspace_too_small_for_the_priced_split(start, T, H, monkeypatch):
+    """A workspace below what the query asks for: the plain split where its
+    partials fit, with that split's own bits, else a refusal, as before there
+    were prices; never a byte past what was given."""
+    D = 128
+    need = int(_native.lib().mgi_paged_prefill_workspace_bytes(start, T, H, D, _native.MGI_BF16))
+    plain = plain_bytes(start, T, H, D)
+    assert 0 < plain <= need
+    call = prefill_with_workspace(start, T, H, D, torch.bfloat16)
+    rc, full = call(need)
+    assert rc == _native.MGI_OK and torch.isfinite(full).all()
+    rc, out = call(plain)
+    assert rc == _native.MGI_OK
+    rows = (out.double() - full.double()).norm(dim=-1) / full.double().norm(dim=-1)
+    assert rows.max().item() <= 2.0 ** -6  # every row and head: a few half-ulps (2^-9) of outputs and weights
+    for nbytes in (plain - 256 if need > plain else 4096, 16, None):  # need == plain: the priced split wants less
+        rc, out = call(nbytes)
+        assert rc == _native.MGI_EWORKSPACE and torch.isnan(out).all()
+    rc, out = call(need, off=8)
+    assert rc == _native.MGI_EINVAL and torch.isnan(out).all()
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("start,T,H,D,dtype", [(8000, 900, 32, 64, torch.bfloat16), (8000, 900, 32, 64, torch.float16),
+                                               (450, 700, 8, 64, torch.float32)])
+def test_calls_without_a_plain_split_run_unsplit_without_room(start, T, H, D, dtype, monkeypatch):
+    """No workspace, too small or misaligned a one, where only the priced split
+    wants any: the unsplit call's bits, as before there were prices."""
+    need = int(_native.lib().mgi_paged_prefill_workspace_bytes(start, T, H, D, _native.DTYPE_CODES[dtype]))
+    assert need > 0 and (dtype == torch.float32 or plain_bytes(start, T, H, D) == 0)
+    call = prefill_with_workspace(start, T, H, D, dtype)
+    rc, split = call(need)
+    assert rc == _native.MGI_OK
+    outs = [call(None), call(need - 256), call(need, off=8)]
+    monkeypatch.setenv("MINIVLLM_HIP_PREFILL_SPLIT_KEYS", "-1")
+    rc, whole = call(None)
+    assert rc == _native.MGI_OK and not torch.equal(split, whole)
+    for rc, out in outs:
+        assert rc == _native.MGI_OK and torch.equal(out, whole)
+    rows = (split.double() - whole.double()).norm(dim=-1) / whole.double().norm(dim=-1)
+    assert rows.max().item() <= {torch.bfloat16: 2.0 ** -6, torch.float16: 2.0 ** -9, torch.float32: 1e-5}[dtype]
