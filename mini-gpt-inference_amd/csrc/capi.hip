@@ -91,8 +91,9 @@ int64_t split_tokens_for(int64_t B, int64_t H, int64_t D, int64_t S, int64_t M,
 // f32): 2-3 waves per CU are best and within noise of each other; 4 per CU is
 // 1-2% slower, and 5-6 per CU (a partial second round) up to 10% slower. A
 // floor of 64 tokens per wave halves small calls against 256 (B=8 x 256
-// tokens, 16 heads: 16.9 against 34.6 us) and leaves large ones unchanged;
-// 16 and 32 are no better. MINIVLLM_HIP_DECODE_BALANCED=0 turns the mode off,
+// tokens, 16 heads: 16.9 against 34.6 us on this split; the workgroup kernel
+// below takes such calls now, 9 us) and leaves large ones unchanged; 16 and 32
+// are no better. MINIVLLM_HIP_DECODE_BALANCED=0 turns the mode off,
 // MINIVLLM_HIP_BAL_WAVES sets the total wave count and
 // MINIVLLM_HIP_BAL_MIN_TOKENS the floor (tuning).
 constexpr int64_t kBalMinTokens = 64;
@@ -156,13 +157,14 @@ SplitPlan split_plan(int64_t B, int64_t H, int64_t D, int64_t S, int64_t M, int6
 // the kernel is taken where the split is not faster whichever rows are long:
 // one row that fills the table among short ones (the workgroups of that row,
 // one per head, end the call), half of the rows (the long workgroups share CUs
-// unevenly, 1.35 times the mean) and all of them. In us:
+// unevenly, 1.35 times the mean) and all of them. In us, MB of K and V with each
+// head row as wide as the lanes it is given (32, 64, 128 or 256 elements):
 //   workgroups  4.2 and the largest of 0.95 ns per wavefront launched; a long
-//               row's K and V per CU and round of the CUs, 23.5 us/MB (30 at 128
-//               bytes per head row, 40 where the row is no whole number of
-//               128-byte lines, 34-58 by H at head_dim up to 32; 1.6 times with
-//               four wavefronts); and all K and V at 6.2 TB/s (5.4, 3.8; 2.8
-//               and, in f32, 4.0)
+//               row per CU and round of the CUs, 23.5 us/MB (30 for 64 2-byte
+//               elements; 28, or 42 for 2-byte rows of up to 64, where head_dim
+//               leaves lanes empty; 35-58 by H up to 32 elements, 1.35 times that
+//               below 32; 1.6 times with four wavefronts); and everything at 6.2
+//               TB/s (5.4; 5.7, 4.0; 2.8 and, in f32, 4.0)
 //   split       12 and all K and V at 6.7 TB/s, or 1.25 times the filled share
 //               of the lanes of its head groups if that is less; at least 18.5,
 //               or 22 for a few long rows among 8 or more (20 and 26 where heads
@@ -172,57 +174,53 @@ SplitPlan split_plan(int64_t B, int64_t H, int64_t D, int64_t S, int64_t M, int6
 //               f32, or all K and V at 6.7 TB/s; up to 16 wavefronts per CU,
 //               with the longest context half of the table: the widths the
 //               runner pads tables to are within that
-// Measured on MI355X over 1725 shapes (1-256 sequences, 2-32 heads, head_dim
-// 32-256, tables of 32-8192 tokens), each with all rows full, random, one and
+// Measured on MI355X over 2408 shapes (1-256 sequences, 2-32 heads, head_dim
+// 8-256, tables of 32-8192 tokens), each with all rows full, random, one and
 // two full, half full and all short: where this takes the kernel, the split is
-// at most 8 % faster on any of the mixes with a context of half the table (5
-// shapes more than 5 %). Split / workgroups, us, bf16, D = 128: 13 x 16 heads,
-// 1024 tokens, one row full 24.4 / 16.4, all 29.4 / 21.5; 1 x 32, 1024: 19.0 /
-// 15.4; 32 x 16, 256, one partition: 29.2 / 14.5, all contexts 16 tokens: 5.3 /
-// 5.8 (64 x 16: 29.4 / 24.9, and 5.5 / 7.4); D = 32, f32, 4 x 8, 256: 48 / 5.7.
-// Left to the split: 13 x 16, 2048, one row full 24.8 / 28.0; 32 x 32, 1024,
-// half 54.0 / 54.0 and 64 x 16 61.3 / 54.4; D = 64, 64 x 4, 8192, one row full
-// 29.0 / 52.4, all 141 / 103; D = 32, 32 x 4, f32, 8192, one 33.4 / 87.7.
-// Eight wavefronts; four where a context is at most half a step of the eight
-// and where eight would be more than 8 per CU (one partition) or 32 (22 x 22,
-// 29-59: 6.7 against 7.7; 64 x 16, D = 64, one row of 512 full: 9.8 against 12.8).
+// at most 9 % faster on any of the mixes with a full row.
+// Split / workgroups, us, bf16, D = 128: 13 x 16 heads, 1024 tokens, one row full
+// 24.4 / 16.4, all 29.4 / 21.5; 1 x 32, 1024: 19.0 / 15.4; 64 x 16, 256, one
+// partition: 29.4 / 24.9, all contexts 16 tokens: 5.5 / 7.4; D = 32, f32, 4 x 8,
+// 256: 58.7 / 7.8. Left to the split: 13 x 16, 2048, one row full 24.8 / 28.0; 64
+// x 16, 1024, half full 54.4 / 61.3; D = 64, 64 x 4, 8192, one row full 29.0 /
+// 52.4, all 137 / 86; D = 32, 32 x 4, f32, 8192, one 33.4 / 87.7.
+// Eight wavefronts; four where a context is at most half a step of the eight (22 x
+// 22, 29-59: 6.7 against 7.7) and, in tables of one partition, where eight would be
+// more than 8 per CU (64 x 16, 256, one row full: 10.0 against 14.2).
 // MINIVLLM_HIP_DECODE_WG = 0 turns the kernel off, 4 or 8 forces it (tuning
 // and tests; read on every call).
 int wg_waves_for(int64_t B, int64_t H, int64_t D, int64_t S, int64_t M, int64_t eb, bool split) {
   const int forced = env_int("MINIVLLM_HIP_DECODE_WG", -1);
   if (forced >= 0) return forced == 0 ? 0 : forced == 4 ? 4 : 8;
-  const int64_t lph = D <= 32 ? 4 : D <= 64 ? 8 : D <= 128 ? 16 : 32, hpw = 64 / lph;
-  const int64_t tokens = M * S, cus = device_cus(), line = D * eb;
+  const int64_t lph = D <= 32 ? 4 : D <= 64 ? 8 : D <= 128 ? 16 : 32, hpw = 64 / lph, width = 8 * lph;
+  const int64_t tokens = M * S, cus = device_cus();
   const int64_t step_tokens = 8 * hpw * (mgi::kGranuleLoads * 2 / eb);  // one step of eight wavefronts
-  const int waves = tokens <= step_tokens / 2 || B * H * 8 > (split ? 32 : 8) * cus ? 4 : 8;
-  const double row_mb = 2e-6 * (double)tokens * (double)line;  // K and V of one full context and head
+  const int waves = tokens <= step_tokens / 2 || (!split && B * H * 8 > 8 * cus) ? 4 : 8;
+  const double kv_mb = 2e-6 * (double)(tokens * D * eb);        // K and V of one full context and head
+  const double row_mb = 2e-6 * (double)(tokens * width * eb);   // with the lanes head_dim leaves empty
   const double launch_us = 0.95e-3 * (double)(B * H * waves);
-  double us_per_mb = 23.5, tbps = 6.2;
-  if (D <= 32) {
-    us_per_mb = 34.0 + 1.5 * (double)std::min<int64_t>(H, 16);
+  const bool full = D == width, thin = width == 64 && eb == 2;
+  double us_per_mb = full ? (thin ? 30.0 : 23.5) : thin ? 42.0 : 28.0;
+  double tbps = full ? (thin ? 5.4 : 6.2) : thin ? 4.0 : 5.7;
+  if (width == 32) {
+    us_per_mb = (34.0 + 1.5 * (double)std::min<int64_t>(H, 16)) * (full ? 1.0 : 1.35);
     tbps = eb == 2 ? 2.8 : 4.0;
-  } else if (line % 128 != 0) {
-    us_per_mb = 40.0;
-    tbps = 3.8;
-  } else if (line == 128) {
-    us_per_mb = 30.0;
-    tbps = 5.4;
   }
   if (!split) {
-    const double token_us = eb == 4 ? 0.18 : 0.11, all_mb = row_mb * (double)(B * H);
+    const double token_us = eb == 4 ? 0.18 : 0.11, rows = (double)(B * H);
+    if (width > 32 && thin) tbps = full ? 6.2 : 5.7;  // short contexts: the lines two heads share stay cached
     const bool pays = B * H * waves <= 16 * cus && 4.2 + launch_us <= 5.2 + 0.5 * token_us * (double)tokens &&
-                      4.2 + all_mb / tbps <= std::max(5.2 + token_us * (double)tokens, 3.0 + all_mb / 6.7);
+                      4.2 + row_mb * rows / tbps <= std::max(5.2 + token_us * (double)tokens, 3.0 + kv_mb * rows / 6.7);
     return pays ? waves : 0;
   }
   const double long_us = row_mb * us_per_mb * (waves == 8 ? 1.0 : 1.6);
   const double lanes = (double)((H + hpw - 1) / hpw * hpw);
-  const double split_tbps = 6.7 * std::min(1.0, 1.25 * (double)(H * D) / (lanes * 8.0 * (double)lph));
-  const bool sparse = 2.0 * (double)H <= lanes || D < 8 * lph;
+  const double split_tbps = 6.7 * std::min(1.0, 1.25 * (double)(H * D) / (lanes * (double)width));
+  const bool sparse = 2.0 * (double)H <= lanes || !full;
   auto pays = [&](double rows, double spread, double split_floor) {  // `rows` full contexts, the others short
-    const double mb = row_mb * rows * (double)H;
-    const double wg_us =
-        4.2 + std::max({std::ceil(rows * (double)H / (double)cus) * long_us, launch_us, spread * mb / tbps});
-    return wg_us <= std::max(split_floor, 12.0 + mb / split_tbps);
+    const double heads = rows * (double)H;
+    const double wg_us = 4.2 + std::max({std::ceil(heads / (double)cus) * long_us, launch_us, spread * row_mb * heads / tbps});
+    return wg_us <= std::max(split_floor, 12.0 + kv_mb * heads / split_tbps);
   };
   const double floor_us = sparse ? 20.0 : 18.5, few_us = B < 8 ? floor_us : sparse ? 26.0 : 22.0;
   return pays(1.0, 1.0, few_us) && pays(0.5 * (double)B, 1.35, floor_us) && pays((double)B, 1.0, floor_us) ? waves : 0;
@@ -328,9 +326,10 @@ int64_t key_partitions(int64_t start, int64_t T, int64_t rows, int64_t k) {
 // D = 128: 513 / 183; 32 after 3000, 8 heads, D = 32: 122 / 14; 1024 after 1024,
 // 16 heads, D = 64: 138 / 96; 3000 at 0, 4 heads: 201 / 86. The split sums are
 // the closer ones to 64 bits (after 16 000 keys 4e-7 against 2.3e-6, the serial
-// sums' error growing by 1.4e-10 a key); chunks that end past kMaxSplitKeysF32
-// stay unsplit, so that no result moves by more than fp32 results are held to
-// (2.4e-6).
+// sums' error growing by 1.4e-10 a key). Chunks that end past kMaxSplitKeysF32
+// stay unsplit. That is no bound of the kernel (they are slower and less close for
+// it): past it the serial sums differ from the split ones by more than 2.4e-6, and
+// results there were not to move by that much.
 constexpr int64_t kMaxSplitKeysF32 = 15360;
 int64_t prefill_split_keys_f32(int64_t start, int64_t T, int64_t H, int64_t D) {
   const int dp = mgi::prefill_head_dim_bucket(0, (int)D);
@@ -437,8 +436,8 @@ PrefillSplit cheapest_prefill_split(int64_t start, int64_t T, int64_t H, int64_t
 // of at most 32) per CU. The plain split, of the total key tiles over two per
 // CU (at least 2), is taken when a tile's 1.5 us (scaled with head_dim) saves
 // more than the split's 8 us and its partials cost; head dims with a
-// direct-to-LDS kernel then look for a cheaper one. Head_dim a multiple of 8 only (the merge's
-// lane layout); fp32 has its own rule above.
+// direct-to-LDS kernel then look for a cheaper one. Head_dim a multiple of 8 only
+// (the merge's lane layout); fp32 has its own rule above.
 // MINIVLLM_HIP_PREFILL_SPLIT_KEYS = -1 turns it off; > 0 forces that many
 // keys per partition of the 2-byte types, rounded up to 64, without the cost
 // models (tuning and tests; read on every call). plain_only: the plain split

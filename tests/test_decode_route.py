@@ -20,6 +20,9 @@ def waves(B, H, D, tokens, dtype=BF16, S=16, split_tokens=0):
     (64, 4, 32, 32768, BF16), (190, 4, 64, 131072, BF16), (64, 2, 128, 8192, BF16), (32, 4, 64, 8192, F32),
     (13, 4, 32, 8192, F32), (64, 4, 64, 8192, BF16), (64, 2, 128, 4096, F32), (1, 32, 128, 2000, BF16),
     (4, 32, 128, 4000, BF16), (190, 4, 64, 9728, F16),
+    # head dims that leave lanes empty cost as much as those that fill them: 31 us against 62, 69 against 173
+    (13, 32, 8, 8192, BF16), (13, 32, 8, 4096, F32), (64, 16, 8, 4096, BF16), (13, 32, 16, 2048, F32),
+    (32, 8, 40, 2048, BF16), (13, 20, 80, 2048, BF16), (4, 8, 24, 2048, BF16),
     # half of the rows long: 55 us against 65
     (256, 4, 128, 1024, BF16), (64, 16, 128, 1024, BF16), (128, 8, 128, 1024, BF16),
     # too many workgroups for short contexts: 5.4 us against 12 or more
