@@ -287,16 +287,13 @@ class KVCacheCausalSelfAttention(nn.Module):
 
 
 _DECODE_METHODS = ("forward_decode_batch", "_qkv_heads", "_finish", "_decode_attend")
-_OWN_METHODS = tuple(KVCacheCausalSelfAttention.__dict__[n] for n in _DECODE_METHODS)
+decode_fused.own_methods(KVCacheCausalSelfAttention, _DECODE_METHODS)
 
 
 def plain_decode_attention(attn: nn.Module) -> bool:
     """Whether attn.forward_decode_batch is this module's own code over plain
     projections, so its parts may be run one by one (decode_fused)."""
     if type(attn) is not KVCacheCausalSelfAttention or not attn.__dict__.keys().isdisjoint(_DECODE_METHODS):
-        return False
-    cls = KVCacheCausalSelfAttention.__dict__
-    if tuple(cls.get(n) for n in _DECODE_METHODS) != _OWN_METHODS:
         return False
     m = attn._modules
     return decode_fused.plain_linear(m["qkv"]) and decode_fused.plain_linear(m["project"]) \

@@ -55,8 +55,8 @@ class TransformerBlock(nn.Module):
         """Whether forward_decode_batch is this module's own code over plain
         submodules (decode_fused)."""
         m = self._modules
-        if not self.fused_decode_linears or type(self) is not TransformerBlock or not self.__dict__.keys().isdisjoint(_DECODE_METHODS) \
-                or tuple(TransformerBlock.__dict__.get(n) for n in _DECODE_METHODS) != _OWN_METHODS \
+        if not self.fused_decode_linears or type(self) is not TransformerBlock \
+                or not self.__dict__.keys().isdisjoint(_DECODE_METHODS) \
                 or not plain_decode_attention(m["attn"]) or m["attn"].n_embd != width:
             return False
         ffn = m["ffn"]
@@ -112,4 +112,4 @@ class TransformerBlock(nn.Module):
 
 
 _DECODE_METHODS = ("forward_decode_batch", "_mlp", "_plain_decode", "_decode_step")
-_OWN_METHODS = tuple(TransformerBlock.__dict__[n] for n in _DECODE_METHODS)
+decode_fused.own_methods(TransformerBlock, _DECODE_METHODS)

@@ -52,41 +52,51 @@ def ops_for(x: Tensor):
     return ops if hasattr(ops, "decode_linear") else None
 
 
-def plain(m: nn.Module, cls: type) -> bool:
-    """Whether calling m runs cls's own forward and nothing else."""
-    return type(m) is cls and cls.forward is _FORWARD[cls] and cls.__call__ is _CALL and not m._forward_hooks \
-        and not m._forward_pre_hooks and "forward" not in m.__dict__
-
-
 def unpatched() -> bool:
-    """Whether the functions those forwards end in are the ones this module was
-    imported with."""
-    return nn.Module._call_impl is _CALL_IMPL and all(getattr(F, n) is f for n, f in _FUNCTIONS.items())
+    """Whether the methods and torch functions the fused calls stand for are the
+    ones this package was imported with (once per step: they belong to classes
+    and modules, not to a model)."""
+    for owner, name, function in _OWN:
+        if getattr(owner, name) is not function:
+            return False
+    return True
 
 
-def plain_params(m: nn.Module, bias: tuple) -> bool:
-    """Whether m.weight and m.bias are m's own parameters (of one of the types
-    ``bias`` for the bias), not attributes or buffers put in their place."""
-    p = m._parameters
-    return type(p.get("weight")) is nn.Parameter and "bias" in p and type(p["bias"]) in bias \
-        and m.__dict__.keys().isdisjoint(_NAMES)
+def own_methods(cls: type, names: tuple[str, ...]) -> None:
+    """Adds cls's methods to what unpatched checks."""
+    _OWN.extend((cls, n, getattr(cls, n)) for n in names)
+
+
+def plain(m: nn.Module, cls: type) -> bool:
+    """Whether calling m runs cls's forward and nothing else, on parameters where
+    it has any: no hooks, and no forward, weight or bias in m's own dict."""
+    d = m.__dict__
+    return type(m) is cls and not d["_forward_hooks"] and not d["_forward_pre_hooks"] \
+        and "forward" not in d and "weight" not in d and "bias" not in d
 
 
 def plain_linear(m: nn.Module) -> bool:
-    return plain(m, nn.Linear) and plain_params(m, (nn.Parameter, type(None)))
+    if not plain(m, nn.Linear):
+        return False
+    p = m._parameters
+    return type(p.get("weight")) is nn.Parameter and "bias" in p and type(p["bias"]) in _PARAMS
 
 
 def plain_norm(m: nn.Module, width: int) -> bool:
-    return plain(m, nn.LayerNorm) and m.normalized_shape == (width,) and plain_params(m, (nn.Parameter,))
+    if not plain(m, nn.LayerNorm) or m.normalized_shape != (width,):
+        return False
+    p = m._parameters
+    return type(p.get("weight")) is nn.Parameter and type(p.get("bias")) is nn.Parameter
 
 
 def idle_dropout(m: nn.Module) -> bool:
     return plain(m, nn.Dropout) and not (m.training and m.p > 0.0)
 
 
-_NAMES = ("weight", "bias")
-_CALL, _CALL_IMPL = nn.Module.__call__, nn.Module._call_impl
-# A forward from elsewhere than its class's module was patched before this import: nothing equals None.
-_FORWARD = {cls: cls.forward if cls.forward.__module__ == cls.__module__ else None
-            for cls in (nn.Linear, nn.LayerNorm, nn.GELU, nn.Dropout, nn.Sequential, FeedForward)}
-_FUNCTIONS = {n: getattr(F, n) for n in ("linear", "layer_norm", "gelu", "dropout")}
+_PARAMS = (nn.Parameter, type(None))
+_OWN = [(nn.Module, "__call__", nn.Module.__call__), (nn.Module, "_call_impl", nn.Module._call_impl)]
+_OWN += [(F, n, getattr(F, n)) for n in ("linear", "layer_norm", "gelu", "dropout")]
+for _cls in (nn.Linear, nn.LayerNorm, nn.GELU, nn.Dropout, nn.Sequential, FeedForward):
+    # A forward from elsewhere than its class's module was patched before this import: nothing is None.
+    _OWN += [(_cls, "forward", _cls.forward if _cls.forward.__module__ == _cls.__module__ else None),
+             (_cls, "__call__", nn.Module.__call__)]

@@ -9,6 +9,7 @@ import torch.nn.functional as F
 from torch import nn
 
 from minivllm import decode_fused
+from minivllm.attention import KVCacheCausalSelfAttention
 from minivllm.block import TransformerBlock
 from minivllm.feed_forward import FeedForward
 from minivllm.model import MiniGPT
@@ -36,29 +37,42 @@ def test_the_attention_backend_does_not_choose(backend):
 
 
 @pytest.mark.parametrize("cls", [nn.Linear, nn.LayerNorm, nn.GELU, nn.Dropout, nn.Sequential, FeedForward])
-def test_a_replaced_class_method_is_called(block, cls, monkeypatch):
+def test_a_replaced_class_method_is_called(cls, monkeypatch):
     """A forward replaced on the class (as quantisers and profilers do) runs in
     a decode step; so does a replaced __call__."""
     forward = cls.forward
-    monkeypatch.setattr(cls, "forward", lambda self, *a, **kw: forward(self, *a, **kw))
-    assert not block._plain_decode(64)
-    monkeypatch.undo()
-    assert block._plain_decode(64)
-    monkeypatch.setattr(cls, "__call__", lambda self, *a, **kw: forward(self, *a, **kw), raising=False)
-    assert not block._plain_decode(64)
-    monkeypatch.undo()
-    assert block._plain_decode(64)
-
-
-@pytest.mark.parametrize("name", ["linear", "layer_norm", "gelu", "dropout"])
-def test_a_replaced_torch_function_is_called(name, monkeypatch):
     assert decode_fused.unpatched()
-    function = getattr(F, name)
-    monkeypatch.setattr(F, name, lambda *a, **kw: function(*a, **kw))
+    monkeypatch.setattr(cls, "forward", lambda self, *a, **kw: forward(self, *a, **kw))
     assert not decode_fused.unpatched()
     monkeypatch.undo()
-    monkeypatch.setattr(nn.Module, "_call_impl", lambda self, *a, **kw: self.forward(*a, **kw))
+    assert decode_fused.unpatched()
+    monkeypatch.setattr(cls, "__call__", lambda self, *a, **kw: forward(self, *a, **kw), raising=False)
     assert not decode_fused.unpatched()
+    monkeypatch.undo()
+    assert decode_fused.unpatched()
+
+
+@pytest.mark.parametrize("owner,name", [
+    (F, "linear"), (F, "layer_norm"), (F, "gelu"), (F, "dropout"), (nn.Module, "_call_impl"), (nn.Module, "__call__"),
+    (TransformerBlock, "_mlp"), (TransformerBlock, "forward_decode_batch"), (KVCacheCausalSelfAttention, "_qkv_heads"),
+    (KVCacheCausalSelfAttention, "_finish"), (KVCacheCausalSelfAttention, "forward_decode_batch")])
+def test_a_replaced_function_is_called(owner, name, monkeypatch):
+    assert decode_fused.unpatched()
+    function = getattr(owner, name)
+    monkeypatch.setattr(owner, name, lambda *a, **kw: function(*a, **kw))
+    assert not decode_fused.unpatched()
+    monkeypatch.undo()
+    assert decode_fused.unpatched()
+
+
+@pytest.mark.parametrize("path,name", [("attn.project", "forward"), ("ffn", "forward"), ("attn", "_finish"), ("", "_mlp")])
+def test_a_method_replaced_on_one_module_is_called(block, path, name):
+    m = block.get_submodule(path)
+    assert block._plain_decode(64)
+    setattr(m, name, lambda *a, **kw: None)
+    assert not block._plain_decode(64)
+    delattr(m, name)
+    assert block._plain_decode(64)
 
 
 @pytest.mark.parametrize("path", ["attn.project", "ffn.network.0", "ffn.network.2", "layer_norm_1", "layer_norm_2"])
