@@ -105,7 +105,7 @@ class TransformerBlock(nn.Module):
         else:
             p = next_norm._parameters
             pair = ops.decode_linear_norm(u, down["weight"], down["bias"], h, p["weight"], p["bias"], next_norm.eps)
-        return (self._mlp(h), None) if pair is None else pair
+        return (h + net["3"](net["2"](u)), None) if pair is None else pair
 
     def forward(self, x: Tensor) -> Tensor:
         return self._mlp(x + self.attn(self.layer_norm_1(x)))

@@ -11,7 +11,9 @@ from torch import nn
 from minivllm import decode_fused
 from minivllm.attention import KVCacheCausalSelfAttention
 from minivllm.block import TransformerBlock
+from minivllm.decode_batch_metadata import DecodeBatchMetadata
 from minivllm.feed_forward import FeedForward
+from minivllm.kv_block_pool import KVBlockPool
 from minivllm.model import MiniGPT
 
 
@@ -99,3 +101,55 @@ def test_a_linear_without_bias_stays_plain(block):
     assert block._plain_decode(64)
     block.attn.project.bias = nn.Parameter(torch.zeros(64))
     assert block._plain_decode(64)
+
+
+class TorchOps:
+    """The binding's two calls in PyTorch, refusing those whose weight is in ``refused``."""
+
+    def __init__(self, refused=()):
+        self.refused = {id(w) for w in refused}
+
+    def decode_linear(self, x, w, bias, gelu):
+        if id(w) in self.refused:
+            return None
+        y = F.linear(x, w, bias)
+        return F.gelu(y) if gelu else y
+
+    def decode_linear_norm(self, x, w, bias, residual, ln_w, ln_b, eps):
+        if id(w) in self.refused:
+            return None
+        h = residual if x is None else F.linear(x, w, bias) + residual
+        return h, None if ln_w is None else F.layer_norm(h, (h.shape[-1],), ln_w, ln_b, eps)
+
+
+@pytest.mark.parametrize("refused", [(), ("attn.qkv",), ("attn.project",), ("ffn.network.0",), ("ffn.network.2",),
+                                     ("attn.qkv", "ffn.network.0", "ffn.network.2")])
+def test_step_with_layers_the_kernels_do_not_take(block, refused):
+    """A block's fused step, each of its layers refused in turn, against the
+    block's own PyTorch calls: the same output and appended KV, and no layer
+    made twice."""
+    g = torch.Generator().manual_seed(1)
+    x = torch.randn((3, 1, 64), generator=g)
+    ctx, tables = torch.tensor([5, 9, 1]), torch.tensor([[2, -1], [0, 3], [1, -1]])
+    slots = tables[torch.arange(3), (ctx - 1) // 8] * 8 + (ctx - 1) % 8
+    meta = DecodeBatchMetadata(positions=ctx - 1, context_lengths=ctx, block_tables=tables, slot_mapping=slots)
+    pools = [KVBlockPool(1, 4, 8, 2, 32) for _ in range(2)]
+    for p in pools:
+        p.k.copy_(torch.randn(p.k.shape, generator=torch.Generator().manual_seed(2)))
+        p.v.copy_(torch.randn(p.v.shape, generator=torch.Generator().manual_seed(3)))
+    after = nn.LayerNorm(64)
+    ops = TorchOps([block.get_submodule(p).weight for p in refused])
+    calls = []
+    for p in ("attn.qkv", "attn.project", "ffn.network.0", "ffn.network.2"):
+        block.get_submodule(p).register_forward_hook(lambda *a, p=p: calls.append(p))
+    with torch.no_grad():
+        want = block.forward_decode_batch(x, metadata=meta, kv_pool=pools[0], layer_idx=0)
+        assert calls == ["attn.qkv", "attn.project", "ffn.network.0", "ffn.network.2"]
+        calls.clear()
+        out, normed = block._decode_step(ops, x, None, after, meta, pools[1], 0)
+    torch.testing.assert_close(out, want, rtol=1e-6, atol=1e-6)
+    assert torch.equal(pools[0].k, pools[1].k) and torch.equal(pools[0].v, pools[1].v)
+    if normed is not None:
+        torch.testing.assert_close(normed, after(out), rtol=1e-6, atol=1e-6)
+    # Without the fused sum after the attention, the MLP is the block's own.
+    assert calls == (["attn.project", "ffn.network.0", "ffn.network.2"] if refused == ("attn.project",) else list(refused))
