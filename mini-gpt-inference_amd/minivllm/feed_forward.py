@@ -1,5 +1,6 @@
 """Position-wise MLP (minivllm/feed_forward.py:3-28): Linear(C, 4C) -> GELU ->
-Linear(4C, C) -> Dropout. Dense GEMMs stay on PyTorch (hipBLASLt)."""
+Linear(4C, C) -> Dropout, as PyTorch calls (hipBLASLt). Decode steps of up to 64
+bf16 or f16 rows run its layers through decode_fused instead."""
 from __future__ import annotations
 
 from torch import Tensor, nn
