@@ -335,6 +335,11 @@ int mgi_decode_linear_norm(void* out, void* norm, const void* x, const void* wei
                            float ln_eps, int dtype, int64_t B, int64_t N, int64_t K,
                            void* workspace, size_t workspace_bytes, void* stream);
 
+/* Whether mgi_decode_linear_norm takes these sizes (K = 0: the LayerNorm
+ * alone) and callers with other calls for them at hand should make this one, as
+ * measured against PyTorch's. */
+int mgi_decode_linear_norm_pays(int64_t B, int64_t N, int64_t K);
+
 /* Workspace bytes mgi_decode_linear_norm needs for these sizes. */
 size_t mgi_decode_linear_norm_workspace_bytes(int64_t B, int64_t N, int64_t K);
 

@@ -994,6 +994,20 @@ int mgi_decode_linear_pays(int64_t B, int64_t N, int64_t K, int gelu) {
   return gelu || B <= 48 || K <= 1536;
 }
 
+// More than 32 rows of more than 12 288 go to PyTorch's linear: a split's x then
+// takes 128 KiB of LDS, one workgroup per CU, and there are 13 and more splits.
+// Measured on MI355X (us, before these calls / with them / without them past that
+// line): a block's step of dim 4096 (K = 16 384), 40 rows 168 / 177 / 158, 64 rows 181
+// / 189 / 172; dim 3072 (K = 12 288) 144 / 131 and 150 / 146, kept; dim 4096, 32 rows
+// 160 / 144.
+int mgi_decode_linear_norm_pays(int64_t B, int64_t N, int64_t K) {
+  using namespace mgi;
+  if (B < 1 || B > kLinearMaxRows || N < 4 || N % 4 != 0 || N > kReduceMaxN || K < 0 || K % 64 != 0 ||
+      K >= (int64_t(1) << 30))
+    return 0;
+  return B <= 32 || K <= 12288;
+}
+
 size_t mgi_decode_linear_norm_workspace_bytes(int64_t B, int64_t N, int64_t K) {
   if (B <= 0 || N <= 0 || K <= 0) return 0;
   return (size_t)(linear_splits(K, nullptr) * B * N * 4);

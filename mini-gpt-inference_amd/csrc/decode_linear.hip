@@ -202,8 +202,8 @@ __global__ void __launch_bounds__(64 * kWaves, 2) decode_linear_resident(const L
 // 13.8 and 29.3 / 19.0; to 4096 columns (replayed, weights from memory): K = 4096,
 // 24.2 / 14.6 and 24.0 / 17.6; K = 16 384, 40.1 / 39.1. More than 32 rows of more
 // than 8192 hold one workgroup per CU (128 KiB of x): 40 rows, K = 10 240, to 2560,
-// 28.7 / 31.4, K = 16 384, to 4096, 33 rows 45.8 / 62.4, kept as the PyTorch calls
-// are three launches. Walking all of K per workgroup (128 workgroups, residual
+// 28.7 / 31.4, K = 16 384, to 4096, 33 rows 45.8 / 62.4 (mgi_decode_linear_norm_pays).
+// Walking all of K per workgroup (128 workgroups, residual
 // in the epilogue, no second launch) took 17.8 and 38.8 for K = 8192.
 constexpr int kSplitWaves = 4;
 constexpr int kSplitN = kSplitWaves * kTileN;

@@ -218,8 +218,6 @@ bool linear_ok(const c10::optional<at::Tensor>& t, const at::Tensor& x, int64_t 
 }
 void* ptr(const c10::optional<at::Tensor>& t) { return t ? t->data_ptr() : nullptr; }
 
-constexpr int64_t kLinearRows = 64;
-
 // decode_linear(x, weight, bias, gelu): act(x W^T + bias) for x [B, 1, K] -> [B,
 // 1, N]; None when the kernel does not take the call, or PyTorch's calls are the
 // faster ones (the caller then makes those).
@@ -239,8 +237,8 @@ py::object decode_linear(const at::Tensor& x, const at::Tensor& w, const c10::op
 
 // decode_linear_norm(x, weight, bias, residual, ln_weight, ln_bias, ln_eps) ->
 // (h, LN(h)) with h = x W^T + bias + residual, or (h, None) without the
-// LayerNorm pair; None when the call is not one the kernel takes. With x and
-// weight None: (residual, LN(residual)).
+// LayerNorm pair; None when the kernel does not take the call, or PyTorch's calls
+// are the faster ones. With x and weight None: (residual, LN(residual)).
 py::object decode_linear_norm(const c10::optional<at::Tensor>& x, const c10::optional<at::Tensor>& w,
                               const c10::optional<at::Tensor>& bias, const at::Tensor& residual,
                               const c10::optional<at::Tensor>& ln_w, const c10::optional<at::Tensor>& ln_b,
@@ -249,18 +247,15 @@ py::object decode_linear_norm(const c10::optional<at::Tensor>& x, const c10::opt
   if (!r.is_cuda() || r.dim() != 3 || r.size(1) != 1 || x.has_value() != w.has_value()) return py::none();
   const int64_t B = r.size(0), N = r.size(2);
   const int dt = dtype_code(r.scalar_type());
-  if ((dt != MGI_BF16 && dt != MGI_F16) || B < 1 || B > kLinearRows || N < 4 || N % 4 != 0 || N > 4096 ||
-      ln_w.has_value() != ln_b.has_value() || (!x && !ln_w))
-    return py::none();
+  if ((dt != MGI_BF16 && dt != MGI_F16) || ln_w.has_value() != ln_b.has_value() || (!x && !ln_w)) return py::none();
   int64_t K = 0;
   if (x) {
     if (x->dim() != 3 || x->size(0) != B || x->size(1) != 1 || w->dim() != 2) return py::none();
     K = x->size(2);
-    if (K < 64 || K % 64 != 0 || w->size(0) != N || w->size(1) != K || !linear_ok(*x, r, B * K) ||
-        !linear_ok(*w, r, N * K))
+    if (K < 1 || w->size(0) != N || w->size(1) != K || !linear_ok(*x, r, B * K) || !linear_ok(*w, r, N * K))
       return py::none();
   }
-  if (!linear_ok(r, r, B * N) || !linear_ok(bias, r, N) || !linear_ok(ln_w, r, N) || !linear_ok(ln_b, r, N))
+  if (!mgi_decode_linear_norm_pays(B, N, K) || !linear_ok(r, r, B * N) || !linear_ok(bias, r, N) || !linear_ok(ln_w, r, N) || !linear_ok(ln_b, r, N))
     return py::none();
   at::Tensor out, norm, ws;
   size_t ws_bytes = 0;

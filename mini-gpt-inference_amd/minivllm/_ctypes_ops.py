@@ -240,25 +240,23 @@ def decode_linear_norm(x: torch.Tensor | None, w: torch.Tensor | None, bias: tor
                        residual: torch.Tensor, ln_w: torch.Tensor | None, ln_b: torch.Tensor | None, ln_eps: float):
     """(h, LN(h)) with h = x W^T + bias + residual, or (h, None) without the
     LayerNorm pair; without x and w (residual, LN(residual)). None when the call
-    is not one the kernel takes."""
+    is not one to make."""
     r = residual
     if not r.is_cuda or r.ndim != 3 or r.shape[1] != 1 or r.dtype not in (torch.bfloat16, torch.float16) \
             or (x is None) != (w is None) or (ln_w is None) != (ln_b is None) or (x is None and ln_w is None):
         return None
     b, n = r.shape[0], r.shape[2]
-    if not 1 <= b <= 64 or not 4 <= n <= 4096 or n % 4 != 0:
-        return None
     k = 0
     if x is not None:
         if x.ndim != 3 or x.shape[0] != b or x.shape[1] != 1 or w.ndim != 2:
             return None
         k = x.shape[2]
-        if k < 64 or k % 64 != 0 or tuple(w.shape) != (n, k) or not _linear_ok(x, r, b * k) \
-                or not _linear_ok(w, r, n * k):
+        if k < 1 or tuple(w.shape) != (n, k) or not _linear_ok(x, r, b * k) or not _linear_ok(w, r, n * k):
             return None
-    if not _linear_ok(r, r, b * n) or not all(_linear_ok(t, r, n) for t in (bias, ln_w, ln_b)):
-        return None
     lib = _native.lib()
+    if not lib.mgi_decode_linear_norm_pays(b, n, k) or not _linear_ok(r, r, b * n) \
+            or not all(_linear_ok(t, r, n) for t in (bias, ln_w, ln_b)):
+        return None
     out = norm = ws = None
     ws_bytes = 0
     if x is not None:

@@ -43,6 +43,7 @@ EXPORTED_SYMBOLS = (
     "mgi_decode_linear",
     "mgi_decode_linear_pays",
     "mgi_decode_linear_norm",
+    "mgi_decode_linear_norm_pays",
     "mgi_decode_linear_norm_workspace_bytes",
 )
 
@@ -133,6 +134,8 @@ def _declare(lib: ctypes.CDLL) -> None:
         _i64, _i64, _i64,                  # B N K
         _p, ctypes.c_size_t, _p,           # workspace, bytes, stream
     ]
+    lib.mgi_decode_linear_norm_pays.restype = _i
+    lib.mgi_decode_linear_norm_pays.argtypes = [_i64, _i64, _i64]
     lib.mgi_decode_linear_norm_workspace_bytes.restype = ctypes.c_size_t
     lib.mgi_decode_linear_norm_workspace_bytes.argtypes = [_i64, _i64, _i64]
 

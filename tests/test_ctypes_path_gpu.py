@@ -80,7 +80,8 @@ def test_decode_linear_calls_are_bit_identical_and_take_the_same(dtype):
               (x.cpu(), w, None, False), (make(65, 1, 128), w, None, False), (make(64, 1, 1600), make(64, 1600), None, False)]
     norm = [(x, w, bias, r, lw, lb, 1e-5), (x, w, None, r, None, None, 0.0), (None, None, None, r, lw, lb, 1e-5),
             (x, None, None, r, lw, lb, 1e-5), (x, w, None, r, lw, None, 1e-5), (None, None, None, r, None, None, 0.0),
-            (x, w, None, r[:4], None, None, 0.0), (odd, w, None, r, None, None, 0.0), (x, w, None, r, lw.float(), lb, 0.0)]
+            (x, w, None, r[:4], None, None, 0.0), (make(33, 1, 12352), make(64, 12352), None, make(33, 1, 64), lw, lb, 1e-5),
+            (x[..., :100].contiguous(), w[:, :100].contiguous(), None, r, None, None, 0.0), (odd, w, None, r, None, None, 0.0), (x, w, None, r, lw.float(), lb, 0.0)]
     taken = 0
     with torch.inference_mode():
         for fn, calls in (("decode_linear", linear), ("decode_linear_norm", norm)):

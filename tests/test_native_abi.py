@@ -388,6 +388,14 @@ def test_decode_linear_sizes_that_pay(B, N, K, gelu, pays):
     assert _native.lib().mgi_decode_linear_pays(B, N, K, gelu) == pays
 
 
+@pytest.mark.parametrize("B,N,K,pays", [
+    (64, 2048, 8192, 1), (64, 3072, 12288, 1), (32, 4096, 16384, 1), (33, 4096, 16384, 0), (64, 4096, 12352, 0),
+    (64, 4096, 4096, 1), (1, 4, 64, 1), (64, 4096, 0, 1), (65, 512, 512, 0), (0, 512, 512, 0), (8, 514, 512, 0),
+    (8, 4100, 512, 0), (8, 0, 512, 0), (8, 512, 100, 0), (8, 512, -64, 0), (8, 512, 1 << 30, 0)])
+def test_decode_linear_norm_sizes_that_pay(B, N, K, pays):
+    assert _native.lib().mgi_decode_linear_norm_pays(B, N, K) == pays
+
+
 def test_decode_linear_entries_reject_bad_arguments():
     """Every argument error is found on the host (made-up addresses, no device
     work): the status, and a message for it."""
