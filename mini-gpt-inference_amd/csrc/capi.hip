@@ -320,7 +320,15 @@ int64_t key_partitions(int64_t start, int64_t T, int64_t rows, int64_t k) {
 // CU's share of all tiles and half a chain; a workgroup adds about 2 us, the
 // split 8 us (merge launch, tail) and its partials written and read back at
 // 5 TB/s. The cheapest partition length is taken when it beats no split by a
-// tenth.
+// tenth. Head dims above 64 (one workgroup per CU, whose 128 KiB of LDS no second
+// one fits beside) weigh it against no split more closely: 3 us more for the split
+// (7 with one-tile partitions on more workgroups than CUs), and no split its longest
+// chain, or past one workgroup per CU the share and an eighth of that chain, or half
+// of it where a head's query tiles fill half its XCD's CUs or less, so that several
+// heads' longest chains start late; by a twentieth (without / with, kept unsplit:
+// 450 rows after 64, 32 heads, D = 96: 67 / 78; 450 after 450, D = 128: 124 / 138;
+// 1900 at 0, 16 heads: 238 / 275; 2000 after 450: 404 / 437; 256 after 64, 32 heads,
+// D = 96: 39 / 43).
 // Measured on MI355X (us, without / with): 700 rows after 450, 8 heads, D = 64:
 // 67 / 30; 512 at 0: 32 / 16; 100 after 1000: 66 / 16; 256 after 4096, 16 heads,
 // D = 128: 513 / 183; 32 after 3000, 8 heads, D = 32: 122 / 14; 1024 after 1024,
@@ -352,6 +360,11 @@ int64_t prefill_split_keys_f32(int64_t start, int64_t T, int64_t H, int64_t D) {
       best_us = us;
       best = 64 * k;
     }
+  }
+  if (dp == 128 && best > 0) {
+    const double late = 16 * nq > (int64_t)cus ? 0.12 : 0.5, n = (double)longest;
+    const double whole_us = 4.0 + tile_us * ((double)(nq * H) <= cus ? n : std::max(n, share + late * n));
+    if (best_us + (best == 64 && share * cus > cus ? 7.0 : 3.0) >= 0.95 * whole_us) return 0;
   }
   return best;
 }

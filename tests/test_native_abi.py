@@ -427,3 +427,15 @@ def test_decode_linear_entries_reject_bad_arguments():
     assert norm(nbytes=need - 1) == WORKSPACE and norm(ws=None) == WORKSPACE
     assert lib.mgi_decode_linear_norm_workspace_bytes(64, 4096, 16384) == 16 * 64 * 4096 * 4
     assert [lib.mgi_decode_linear_norm_workspace_bytes(*s) for s in ((0, 64, 64), (4, 0, 64), (4, 64, 0))] == [0, 0, 0]
+
+
+@pytest.mark.parametrize("start,T,H,D,dtype,parts", [
+    # fp32: unsplit where the chains already end together (with / without the split, us: 78 / 67, 138 / 124, 437 / 404,
+    # 43 / 39, 275 / 238), split where they do not (185 / 224, 183 / 513)
+    (64, 450, 32, 96, 0, 0), (450, 450, 32, 128, 0, 0), (450, 2000, 16, 128, 0, 0), (64, 256, 32, 96, 0, 0),
+    (0, 1900, 16, 128, 0, 0),
+    (0, 1024, 32, 96, 0, 4), (4096, 256, 16, 128, 0, 14)])
+def test_prefill_splits_near_the_line(start, T, H, D, dtype, parts, monkeypatch):
+    monkeypatch.delenv("MINIVLLM_HIP_PREFILL_SPLIT_KEYS", raising=False)
+    n = T * H * parts
+    assert _native.lib().mgi_paged_prefill_workspace_bytes(start, T, H, D, dtype) == -(-n * D * 4 // 256) * 256 + n * 8
