@@ -481,7 +481,13 @@ PrefillSplit prefill_split(int64_t start, int64_t T, int64_t H, int64_t D, int d
     if (split_us < (double)longest * tile_us && parts <= kMaxGridYZ)
       plain = {64 * k, (T + 127) / 128 * H * parts >= device_cus() && k >= 32 ? 1422 : 412};
   }
-  return T > 32 && (dp == 64 || dp == 128) && !plain_only ? cheapest_prefill_split(start, T, H, D, plain) : plain;
+  // A plain split of a chunk whose 128-row tiles alone fill the CUs stays: it only
+  // trims the longest chains, and the short partitions left over fill in behind
+  // them, which the prices (of whole rounds) miss: 4000 rows after 4096, 8 heads,
+  // 125 us against 141 with the split priced lowest (D = 64: 91 / 97).
+  const bool trimmed = plain.keys > 0 && (T + 127) / 128 * H >= device_cus();
+  const bool priced = T > 32 && (dp == 64 || dp == 128) && !plain_only && !trimmed;
+  return priced ? cheapest_prefill_split(start, T, H, D, plain) : plain;
 }
 
 struct PrefillWorkspace {

@@ -434,7 +434,9 @@ def test_decode_linear_entries_reject_bad_arguments():
     # 43 / 39, 275 / 238), split where they do not (185 / 224, 183 / 513)
     (64, 450, 32, 96, 0, 0), (450, 450, 32, 128, 0, 0), (450, 2000, 16, 128, 0, 0), (64, 256, 32, 96, 0, 0),
     (0, 1900, 16, 128, 0, 0),
-    (0, 1024, 32, 96, 0, 4), (4096, 256, 16, 128, 0, 14)])
+    (0, 1024, 32, 96, 0, 4), (4096, 256, 16, 128, 0, 14),
+    # bf16: 128-row tiles that fill the CUs keep the plain split, two partitions (141 / 125)
+    (4096, 4000, 8, 128, 1, 2), (4096, 4000, 8, 64, 1, 2)])
 def test_prefill_splits_near_the_line(start, T, H, D, dtype, parts, monkeypatch):
     monkeypatch.delenv("MINIVLLM_HIP_PREFILL_SPLIT_KEYS", raising=False)
     n = T * H * parts
