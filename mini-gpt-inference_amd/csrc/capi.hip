@@ -387,8 +387,9 @@ struct PrefillSplit {
 // tiles cost more when H is no multiple of 8, as a head's workgroups then
 // spread over the XCDs. `plain`, the split with one partition length (total
 // tiles over two per CU), stays unless a candidate is 7 % cheaper: nearer
-// than that the estimates don't tell them apart. Measured on MI355X, plain
-// / this (us, bf16, D = 128, replayed from a graph): 300 rows after 15 000, 32
+// than that the estimates don't tell them apart (the worst of 237 shapes: 8 %
+// slower, 1900 rows after 4096, 4 heads, D = 64: 31.0 / 33.6). Measured on MI355X,
+// plain / this (us, bf16, D = 128, replayed from a graph): 300 rows after 15 000, 32
 // heads: 177 / 136; 640 after 15 000: 214 / 195; 400 after 6000, 20 heads:
 // 87 / 59; 900 after 3000, 16 heads: 59 / 55; 450 after 5000, 32 heads: 66 /
 // 63; 1100 after 5000, 12 heads: 80 / 66; 500 after 10 000, 12 heads, D = 64:
